@@ -16,7 +16,7 @@ int gd_hip_launch_linear_bf16(hipStream_t stream, const void *x, const void *w, 
                               int kn_vector_ok, int store_vector_ok, int min_workgroups, const gd_hip_rope_epilogue *rope,
                               int wide_mode, int *family);
 int gd_hip_launch_linear_f32(hipStream_t stream, const void *x, const void *w, const void *bias, void *y,
-                             const gd_hip_linear_params *params);
+                             const gd_hip_linear_params *params, int compute_units);
 
 static gd_status project_full(gd_backend *backend, const gd_backend_matrix_view *x, const gd_backend_matrix_view *w,
                               const gd_backend_vector_view *bias, const gd_backend_matrix_view *residual,
@@ -96,7 +96,7 @@ static gd_status project_full(gd_backend *backend, const gd_backend_matrix_view 
         backend->last_linear_family = GD_HIP_LINEAR_FAMILY_F32;
         return gd_hip_finish_op(backend, gd_hip_launch_linear_f32(
             backend->stream, gd_hip_matrix_ptr(x), gd_hip_matrix_ptr(w), bias != NULL ? gd_hip_vector_ptr(bias) : NULL,
-            gd_hip_matrix_ptr(y), &p));
+            gd_hip_matrix_ptr(y), &p, backend->compute_units));
     }
     /* 16-byte fragment loads: x rows always, w rows when K-contiguous, the norm weight */
     vec = (K % 8u) == 0u && ((x->offset | x->row_bytes) & 15u) == 0u &&

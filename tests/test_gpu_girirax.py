@@ -54,6 +54,23 @@ def test_projections_of_both_types(backend, gda, arena, dtype, M, N, K):
             _near(half.read_float(), value * act, dtype)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 32), (7, 70, 96), (32, 33, 128), (33, 64, 64), (65, 130, 160), (16, 16500, 64), (1030, 1000, 96),
+                                   (1025, 1090, 32)])
+def test_32_bit_projections_on_the_matrix_cores(backend, gda, arena, M, N, K):
+    """Edges of the 32 x 32 (K split four ways) and 64 x 64 tiles; plain with a bias, and gated."""
+    rng = np.random.default_rng(M + N + K)
+    x, xv = _put(arena, F32, rng.standard_normal((M, K)))
+    w, wv = _put(arena, F32, rng.standard_normal((2 * N, K)) / np.sqrt(K))
+    b, bv = _put(arena, F32, rng.standard_normal(2 * N))
+    y = arena.alloc((M, 2 * N), F32).write(np.full((M, 2 * N), np.nan, np.float32))
+    want = xv @ wv.T + bv
+    backend.fused_linear(x, w, b, None, None, y, True, 1, 0)
+    _near(y.read(), want, F32)
+    half, gate = arena.alloc((M, N), F32).write(np.full((M, N), np.nan, np.float32)), want[:, N:]
+    backend.fused_linear(x, w, b, None, None, half, True, 1, 0, epilogue=1)
+    _near(half.read(), want[:, :N] * gate / (1 + np.exp(-gate)), F32)
+
+
 def test_big_tiles_and_unsupported_forms(backend, gda, arena):
     """Enough 256 x 256 tiles for every compute unit, with ragged edges, plain and gated; and what BF16 does not have."""
     rng = np.random.default_rng(5)
