@@ -30,11 +30,13 @@ static void launch_wide_half(hipStream_t stream, const void *x, const void *w, c
         (const gd_elem *)x, (const gd_elem *)w, (const gd_elem *)bias, (const gd_elem *)residual, (gd_elem *)y, p, n_tiles);
 }
 
-/* persistent form: K = 2048 behind an rms_norm, at most 8 tiles per workgroup, one workgroup per compute unit */
-template <int NT, int MT, int EPI>
-static void launch_persistent(hipStream_t stream, const void *x, const void *w, const void *bias, const void *residual,
+/* persistent form: at most 8 tiles per workgroup, one workgroup per compute unit; outputs in tiles of 16 * NT columns (paired
+ * epilogues: 8 * NT), the last one perhaps not full.  F16: K = 2048 behind an rms_norm.  false: nothing launched, because fewer
+ * than min_tiles workgroups would stream */
+template <int NT, int MT, int PMAX, int EPI, int PRO>
+static bool launch_persistent(hipStream_t stream, const void *x, const void *w, const void *bias, const void *residual,
                               const void *norm_w, void *y, const gd_hip_linear_params &p, const gd_hip_rope_epilogue &rope,
-                              uint32_t units, bool narrow)
+                              uint32_t units, bool narrow, uint32_t min_tiles)
 {
     constexpr bool PAIRED = EPI != GD_WIDE_EPI_PLAIN;
     /* as deep as LDS allows next to the sums of the wavefronts (NT x MT x 8 KB): 8 x RING x 2 KB; an eighth group for
@@ -42,7 +44,7 @@ static void launch_persistent(hipStream_t stream, const void *x, const void *w, 
     constexpr int RING = NT * MT <= 4 ? 7 : 5;
     const uint32_t cols = PAIRED ? 8u * NT : 16u * NT;
     const uint32_t outs = EPI == GD_WIDE_EPI_ROPE ? p.N / 2u : (EPI == GD_WIDE_EPI_SWIGLU ? p.swiglu_cols : p.N);
-    uint32_t n_tiles = outs / cols, tile_w = cols;
+    uint32_t n_tiles = (outs + cols - 1u) / cols, tile_w = cols;
     /* fewer full tiles than compute units (5632 gated outputs: 176 tiles of 32): narrower tiles, one per unit, so
      * that every unit streams its share of the weights (22 columns each; the 3072 rotation pairs of a 6144-row qkv
      * weight: 12 pairs each).  Narrow rope tiles straddle heads: only when half the head size is a power of two. */
@@ -52,13 +54,39 @@ static void launch_persistent(hipStream_t stream, const void *x, const void *w, 
         tile_w = (outs + units - 1u) / units; /* more than half of a tile's columns stay in use */
         n_tiles = (outs + tile_w - 1u) / tile_w;
     }
+    if (n_tiles < min_tiles) return false;
     uint32_t groups = n_tiles < units ? n_tiles : units;
     if ((n_tiles + groups - 1u) / groups > 8u) groups = (n_tiles + 7u) / 8u;
     dim3 grid(groups, (p.M + 16u * MT - 1u) / (16u * MT));
-    gd_linear_wide_persistent_kernel<NT, MT, 4, RING, EPI, 8><<<grid, 512, 0, stream>>>(
+    gd_linear_wide_persistent_kernel<NT, MT, PMAX, RING, EPI, 8, PRO><<<grid, 512, 0, stream>>>(
         (const gd_elem *)x, (const gd_elem *)w, (const gd_elem *)bias, (const gd_elem *)residual,
         (const gd_elem *)norm_w, (gd_elem *)y, p, n_tiles, tile_w, rope);
+    return true;
 }
+
+#if GD_LINEAR_IS_BF16
+/* BF16: the widest column tiles that leave at most a quarter of the compute units without one (with fewer workgroups the
+ * 16-column form streams faster).  Four row tiles keep 32 columns (their sums would not fit beside the ring), and K = 4096 two
+ * row tiles (registers).  Against the 16-column form, which reads x (as many bytes as its weights) for every 16 columns and the
+ * weights for every 16 rows, and against the stream kernel for gated outputs, weights from HBM (us; 4, 16, 32, 64 rows):
+ *   1024 -> 32768 F32 results  15.5, 15.9, 18.1, 22.2 (24.7, 29.1, 53.1, 99.9): 4.3 to 3.0 TB/s
+ *   2048 -> 32768 F32 results  30.1, 29.6, 31.8, 37.2 (37.1, 38.6, 67.3, 121): 4.5 to 3.6 TB/s
+ *   1024 -> 2816 gated         5.1, 5.1, 6.1, 8.7 (5.9, 6.4, 8.6, 14.3);  2048 -> 5632 gated 12.2, 12.8, 14.9, 21.0 (15.9, 16.5, 26.3, 37.1)
+ *   1024 -> 4384               4.6, 4.8, 5.8, 8.3 (6.6, 7.7, 11.0, 17.5);  4096 -> 8448 17.5, 19.1, 22.8, 41.0 (24.1, 31.0, 48.3, 82.8) */
+template <int PMAX, int EPI>
+static bool launch_persistent_rows(hipStream_t stream, const void *x, const void *w, const void *bias, void *y,
+                                   const gd_hip_linear_params &p, const gd_hip_rope_epilogue &rope, uint32_t units)
+{
+    const uint32_t least = units - units / 4u;
+#define GD_P(NT, MT) launch_persistent<NT, MT, PMAX, EPI, GD_HIP_PRO_NONE>(stream, x, w, bias, nullptr, nullptr, y, p, rope, units, true, least)
+    if (p.M <= 16u) return GD_P(4, 1) || GD_P(2, 1);
+    if constexpr (PMAX <= 4) {
+        if (p.M > 32u) return GD_P(2, 4);
+    }
+    return GD_P(4, 2) || GD_P(2, 2);
+#undef GD_P
+}
+#endif
 
 /* Returns 1 when the launch was taken (hipGetLastError() then tells how it went), 0 when this kernel family does
  * not cover the call and the caller goes on to the stream kernel.  Covered: [N,K] weights of at least min_bytes
@@ -83,6 +111,23 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
     const uint32_t ppw = (p.K / 64u + 7u) / 8u; /* pairs of steps per wavefront */
     const int epi = p.rope_head_dim != 0u ? GD_WIDE_EPI_ROPE : (p.swiglu_cols != 0u ? GD_WIDE_EPI_SWIGLU : GD_WIDE_EPI_PLAIN);
     const uint32_t mt = p.M <= 16u ? 1u : (p.M <= 32u ? 2u : 4u);
+#if GD_LINEAR_IS_BF16
+    /* K that the eight wavefronts share in whole pairs of steps: the persistent form; other K and narrower outputs go on */
+    if (tiles != 1u && p.prologue == GD_HIP_PRO_NONE && epi != GD_WIDE_EPI_ROPE) {
+#define GD_R(PMAX, EPI) if (p.K == 512u * PMAX && launch_persistent_rows<PMAX, EPI>(stream, x, w, bias, y, p, rope, units)) return 1
+        if (epi == GD_WIDE_EPI_PLAIN) {
+            GD_R(1, GD_WIDE_EPI_PLAIN);
+            GD_R(2, GD_WIDE_EPI_PLAIN);
+            GD_R(4, GD_WIDE_EPI_PLAIN);
+            GD_R(8, GD_WIDE_EPI_PLAIN);
+        } else {
+            GD_R(2, GD_WIDE_EPI_SWIGLU);
+            GD_R(4, GD_WIDE_EPI_SWIGLU);
+            GD_R(8, GD_WIDE_EPI_SWIGLU);
+        }
+#undef GD_R
+    }
+#endif
     const bool persistent = tiles != 1u; /* "linear_tiles" = 1 asks for the one-tile-per-workgroup form (for comparison) */
 #define GD_W(NT, MT, PMAX, PRO, EPI) \
     do { launch_wide<NT, MT, PMAX, PRO, EPI>(stream, x, w, bias, residual, norm_w, y, p, rope); return 1; } while (0)
@@ -110,7 +155,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
     if (p.prologue != GD_HIP_PRO_RMS_NORM || ppw > 4u) return 0;
     /* K = 2048: the persistent form, where its LDS holds the sums of MT x NT tiles next to the ring */
 #define GD_P(NT, MT, EPI) \
-    do { launch_persistent<NT, MT, EPI>(stream, x, w, bias, residual, norm_w, y, p, rope, units, tiles != 4u); return 1; } while (0)
+    do { launch_persistent<NT, MT, 4, EPI, GD_HIP_PRO_RMS_NORM>(stream, x, w, bias, residual, norm_w, y, p, rope, units, tiles != 4u, 0u); return 1; } while (0)
     if (p.K == 2048u && persistent) {
         if (epi == GD_WIDE_EPI_PLAIN && (p.N % 64u) == 0u && mt <= 2u) {
             if (mt == 1u) GD_P(4, 1, GD_WIDE_EPI_PLAIN);

@@ -521,15 +521,15 @@ gd_linear_wide_half_kernel(const gd_elem *__restrict__ x, const gd_elem *__restr
 }
 
 /*
- * The same projection for matrices with MANY column tiles (rms_norm prologue, K = 512 * PMAX: every wavefront owns
- * exactly PMAX pairs of steps): persistent workgroups.  gridDim.x workgroups share the n_tiles column tiles in
+ * The same projection for matrices with MANY column tiles (K = 512 * PMAX: every wavefront owns exactly PMAX pairs of
+ * steps; PRO: rms_norm prologue (F16) or none (BF16)): persistent workgroups.  gridDim.x workgroups share the n_tiles column tiles in
  * contiguous runs; a workgroup loads and normalises its activation slice ONCE and then walks its tiles with the
  * weight ring running on across tile ends (the first groups of the next tile are in flight while the sums of the
  * current one go through LDS and out), so the stream of a compute unit is interrupted neither by a launch nor by a
  * prologue.  Bias values and positions of all its tiles are copied to LDS up front: the steady state issues no
  * register loads, whose waits would also wait for the ring.  At most TPW tiles per workgroup (host).
  */
-template <int NT, int MT, int PMAX, int RING, int EPI, int TPW>
+template <int NT, int MT, int PMAX, int RING, int EPI, int TPW, int PRO>
 __global__ void __launch_bounds__(512)
 gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__ w,
                                  const gd_elem *__restrict__ bias, const gd_elem *__restrict__ residual,
@@ -544,10 +544,10 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
     constexpr int EPT = (NTO * MT * 256 + 511) / 512;
     constexpr uint32_t COLS = 16u * NT, OUT_COLS = 16u * NTO;
     static_assert(!PAIRED || NT >= 2, "paired epilogues need two column tiles");
-    static_assert(RING >= 3 && RING <= 8 && RING <= NG, "ring depth");
+    static_assert(RING >= 3 && RING <= 8, "ring depth");
     __shared__ __align__(16) unsigned char s_ring[WAVES * RING * 2048];
     __shared__ __align__(16) float s_sum[WAVES * MT * NT * 256];
-    __shared__ float s_part[WAVES][MT][16];
+    __shared__ float s_part[PRO == GD_HIP_PRO_RMS_NORM ? WAVES : 1][MT][16];
     __shared__ gd_elem s_bias[2][TPW * OUT_COLS];
     __shared__ int32_t s_pos[2][16 * MT];
 
@@ -632,7 +632,7 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
     const unsigned char *nb = reinterpret_cast<const unsigned char *>(norm_w) + (size_t)p_begin * 128u;
     gd_elem8 ar[MT][SMAX];
     {
-        gd_elem8 nr[SMAX];
+        gd_elem8 nr[PRO == GD_HIP_PRO_RMS_NORM ? SMAX : 1];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const uint32_t mrow = min(m0 + 16u * mt + (uint32_t)li, p.M - 1u);
@@ -640,9 +640,11 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
 #pragma unroll
             for (int s = 0; s < SMAX; ++s) ar[mt][s] = gd_wide_request16(xb, (uint32_t)s * 64u + xoff);
         }
+        if constexpr (PRO == GD_HIP_PRO_RMS_NORM) {
 #pragma unroll
-        for (int s = 0; s < SMAX; ++s) nr[s] = gd_wide_request16(nb, (uint32_t)s * 64u + (uint32_t)lg * 16u);
-    int first_groups = 0;
+            for (int s = 0; s < SMAX; ++s) nr[s] = gd_wide_request16(nb, (uint32_t)s * 64u + (uint32_t)lg * 16u);
+        }
+        int first_groups = 0;
 #pragma unroll
         for (int g = 0; g < RING; ++g) {
             if (g < total_groups) {
@@ -659,8 +661,10 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int s = 0; s < SMAX; ++s) gd_wide_arrived(ar[mt][s]);
+        if constexpr (PRO == GD_HIP_PRO_RMS_NORM) {
 #pragma unroll
-        for (int s = 0; s < SMAX; ++s) gd_wide_arrived(nr[s]);
+            for (int s = 0; s < SMAX; ++s) gd_wide_arrived(nr[s]);
+        }
         if (has_col) {
             s_bias[0][threadIdx.x] = gd_wide_half_of(rq_b1);
             s_bias[1][threadIdx.x] = gd_wide_half_of(rq_b2);
@@ -669,31 +673,35 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
             s_pos[0][threadIdx.x] = (int32_t)rq_pos;
             s_pos[1][threadIdx.x] = (int32_t)rq_cpos;
         }
-        float ss[MT];
+        if constexpr (PRO == GD_HIP_PRO_RMS_NORM) {
+            float ss[MT];
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            ss[mt] = 0.f;
+            for (int mt = 0; mt < MT; ++mt) {
+                ss[mt] = 0.f;
 #pragma unroll
-            for (int s = 0; s < SMAX; ++s)
+                for (int s = 0; s < SMAX; ++s)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) ss[mt] = fmaf((float)ar[mt][s][e], (float)ar[mt][s][e], ss[mt]);
-            ss[mt] += __shfl_xor(ss[mt], 16, 64);
-            ss[mt] += __shfl_xor(ss[mt], 32, 64);
-            if (lg == 0) s_part[wave][mt][li] = ss[mt];
+                    for (int e = 0; e < 8; ++e) ss[mt] = fmaf((float)ar[mt][s][e], (float)ar[mt][s][e], ss[mt]);
+                ss[mt] += __shfl_xor(ss[mt], 16, 64);
+                ss[mt] += __shfl_xor(ss[mt], 32, 64);
+                if (lg == 0) s_part[wave][mt][li] = ss[mt];
+            }
         }
         /* LDS writes visible (row sums, bias, positions), then the barrier; the ring loads are not waited for */
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if constexpr (PRO == GD_HIP_PRO_RMS_NORM) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            float tot = 0.f;
+            for (int mt = 0; mt < MT; ++mt) {
+                float tot = 0.f;
 #pragma unroll
-            for (int wv = 0; wv < WAVES; ++wv) tot += s_part[wv][mt][li];
-            const float minv = rsqrtf(tot / (float)p.K + p.eps);
+                for (int wv = 0; wv < WAVES; ++wv) tot += s_part[wv][mt][li];
+                const float minv = rsqrtf(tot / (float)p.K + p.eps);
 #pragma unroll
-            for (int s = 0; s < SMAX; ++s)
+                for (int s = 0; s < SMAX; ++s)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    ar[mt][s][e] = (gd_elem)((float)ar[mt][s][e] * (float)nr[s][e] * minv);
+                    for (int e = 0; e < 8; ++e)
+                        ar[mt][s][e] = (gd_elem)((float)ar[mt][s][e] * (float)nr[s][e] * minv);
+            }
         }
     }
 
@@ -772,6 +780,17 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
             if (row >= p.M || !col_used) continue;
             const gd_elem b1 = s_bias[0][ti * (int)OUT_COLS + 16 * j + (rl & 15)];
             const gd_elem b2 = s_bias[1][ti * (int)OUT_COLS + 16 * j + (rl & 15)];
+#if GD_LINEAR_IS_BF16
+            /* F32 up to the one rounding, the gate and the square of relu included */
+            if (p.epilogue != GD_HIP_EPI_NONE) {
+                v1 += (float)b1;
+                if (PAIRED) v2 += (float)b2;
+            }
+            if (EPI == GD_WIDE_EPI_SWIGLU) v1 = gd_lin_gated(v1, v2, p);
+            else v1 = gd_lin_activated(v1, p.flags);
+            if (p.flags & GD_HIP_LINEAR_Y_F32) reinterpret_cast<float *>(y)[(size_t)row * p.ldy + col] = v1;
+            else y[(size_t)row * p.ldy + col] = (gd_elem)v1;
+#else
             gd_elem h1, h2 = (gd_elem)0.f;
             if (p.epilogue == GD_HIP_EPI_BIAS_F32) {
                 h1 = (gd_elem)(v1 + (float)b1);
@@ -811,6 +830,7 @@ gd_linear_wide_persistent_kernel(const gd_elem *__restrict__ x, const gd_elem *_
                     }
                 }
             }
+#endif
         }
         /* the sums have been read: the next tile may overwrite them */
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");

@@ -71,6 +71,26 @@ def test_32_bit_projections_on_the_matrix_cores(backend, gda, arena, M, N, K):
     _near(half.read(), want[:, :N] * gate / (1 + np.exp(-gate)), F32)
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 8200, 512), (16, 4099, 1024), (17, 4099, 1024), (33, 3073, 1024), (65, 12301, 512), (40, 2050, 2048),
+                                   (3, 3100, 4096), (64, 1600, 4096)])
+def test_few_rows_onto_many_columns(backend, gda, arena, M, N, K):
+    """Column tiles of every width, the last one not full, dealt out to persistent workgroups: plain to BF16 and F32, and gated."""
+    rng = np.random.default_rng(M + N + K)
+    x, xv = _put(arena, BF16, rng.standard_normal((M, K)))
+    w, wv = _put(arena, BF16, rng.standard_normal((2 * N, K)) / np.sqrt(K))
+    b, bv = _put(arena, BF16, rng.standard_normal(2 * N))
+    y, wide = arena.alloc((M, 2 * N), BF16), arena.alloc((M, 2 * N), F32)
+    want = xv @ wv.T
+    backend.fused_linear(x, w, b, None, None, y, True, 1, 0)
+    assert backend.linear_last_kernel() == "wide"
+    _near(y.read_float(), want + bv, BF16)
+    backend.matmul_nt(x, w, wide)
+    _near(wide.read_float(), want, F32, factor=3)
+    half, gate = arena.alloc((M, N), BF16), (want + bv)[:, N:]
+    backend.fused_linear(x, w, b, None, None, half, True, 1, 0, epilogue=1)
+    _near(half.read_float(), (want + bv)[:, :N] * gate / (1 + np.exp(-gate)), BF16)
+
+
 def test_big_tiles_and_unsupported_forms(backend, gda, arena):
     """Enough 256 x 256 tiles for every compute unit, with ragged edges, plain and gated; and what BF16 does not have."""
     rng = np.random.default_rng(5)
