@@ -30,7 +30,7 @@ typedef struct gd_extend_rows {
 } gd_extend_rows;
 
 /* A model behind a decoder.  All of these enqueue inside an open step scope and leave logits [rows, vocab] of the
- * decoder's logits type in scratch. */
+ * decoder's logits type in scratch, or where they are to be kept anyway (gd_decoder_logits). */
 typedef struct gd_decoder_model {
     const char *architecture;
     /* packed prompts of every batch row from position 0: logits of each row's last token */
@@ -68,7 +68,8 @@ struct gd_gpt_decoder {
     gd_backend_graph *resident_graph;
     gd_tensor resident_out_ids, resident_out_gaps;
     /* sampling front end (state arena): what the reference's generation loop keeps on the host */
-    gd_tensor last_logits;                 /* [B, V] F16 or F32: logits of the last packed prefill */
+    gd_tensor last_logits;                 /* [B, V] F16 or F32: logits of the last packed prefill, or kept ones of a step */
+    bool keep_logits;                      /* the forward being enqueued may write its logits to last_logits */
     gd_tensor history, hist_len, finished; /* [B, max_seq], [B], [B] I32 */
     gd_tensor sample_state, sample_work;   /* generator + per-row records; [B*V] F32 */
     bool resident_sampling;
@@ -81,6 +82,9 @@ gd_status gd_decoder_session_create(gd_context *ctx, const gd_decoder_model *mod
                                     gd_gpt_decoder **out);
 gd_status gd_decoder_session_allocate(gd_gpt_decoder *d, gd_dtype logits_dtype, bool x0_rows);
 size_t gd_decoder_session_bytes(const gd_gpt_config *cfg, gd_dtype logits_dtype, bool x0_rows);
+
+/* where a forward over n rows puts its logits: last_logits while they are to be kept, scratch otherwise */
+gd_status gd_decoder_logits(gd_gpt_decoder *d, int64_t n, gd_tensor *logits);
 
 static inline size_t gd_pad256(size_t n) { return (n + 255U) & ~(size_t)255U; }
 

@@ -741,17 +741,16 @@ static gd_status scratch_f16(gd_context *ctx, int64_t rows, int64_t cols, gd_ten
 }
 
 /* y = [residual +] bias_mode(prologue(x) @ w) through gd_backend_fused_linear */
-static gd_status fused_project_rows(gd_gpt_decoder *d, int64_t B, const gd_tensor *x, int64_t x_cols,
+/* y [B, n_out] exists */
+static gd_status fused_project_into(gd_gpt_decoder *d, int64_t B, const gd_tensor *x, int64_t x_cols,
                                     const gpt_linear *lin, const gd_tensor *w_override, const gd_tensor *bias,
                                     const gd_tensor *residual, const gd_tensor *norm_w, uint32_t prologue,
-                                    uint32_t epilogue, int64_t n_out, gd_tensor *y)
+                                    uint32_t epilogue, int64_t n_out, const gd_tensor *y)
 {
     gd_backend_matrix_view xm, wm, rm, ym;
     gd_backend_vector_view bv, nv;
     gd_backend_fused_linear_args a;
     const gd_tensor *w = w_override != NULL ? w_override : &lin->weight;
-    gd_status st;
-    TRY(scratch_f16(d->ctx, B, n_out, y));
     mview(x, B, x_cols, &xm);
     mview(w, w->shape[0], w->shape[1], &wm);
     mview(y, B, n_out, &ym);
@@ -764,9 +763,17 @@ static gd_status fused_project_rows(gd_gpt_decoder *d, int64_t B, const gd_tenso
     a.prologue = prologue;
     a.eps = d->cfg.rms_eps;
     a.epilogue = epilogue;
-    st = gd_backend_fused_linear(gd_context_backend(d->ctx), &xm, &wm, &bv, residual != NULL ? &rm : NULL,
-                                 norm_w != NULL ? &nv : NULL, &ym, &a);
-    return st;
+    return gd_backend_fused_linear(gd_context_backend(d->ctx), &xm, &wm, &bv, residual != NULL ? &rm : NULL,
+                                   norm_w != NULL ? &nv : NULL, &ym, &a);
+}
+
+static gd_status fused_project_rows(gd_gpt_decoder *d, int64_t B, const gd_tensor *x, int64_t x_cols,
+                                    const gpt_linear *lin, const gd_tensor *w_override, const gd_tensor *bias,
+                                    const gd_tensor *residual, const gd_tensor *norm_w, uint32_t prologue,
+                                    uint32_t epilogue, int64_t n_out, gd_tensor *y)
+{
+    TRY(scratch_f16(d->ctx, B, n_out, y));
+    return fused_project_into(d, B, x, x_cols, lin, w_override, bias, residual, norm_w, prologue, epilogue, n_out, y);
 }
 
 static gd_status fused_project(gd_gpt_decoder *d, const gd_tensor *x, int64_t x_cols, const gpt_linear *lin,
@@ -847,7 +854,8 @@ static gd_status enqueue_fused_step(gd_gpt_decoder *d, gd_tensor *logits)
         head_lin.weight = d->lm_head;
         head_lin.bias = d->lm_head_bias;
         head_lin.transposed = true;
-        TRY(fused_project(d, &x, Dm, &head_lin, NULL, &d->lm_head_bias, NULL, &d->final_norm_w, 2U, 0U, c->vocab, logits));
+        TRY(gd_decoder_logits(d, B, logits));
+        TRY(fused_project_into(d, B, &x, Dm, &head_lin, NULL, &d->lm_head_bias, NULL, &d->final_norm_w, 2U, 0U, c->vocab, logits));
     }
     return GD_OK;
 }

@@ -563,7 +563,7 @@ static gd_status head(forward *f, const gd_backend_tensor_view *rows, int64_t n,
     gd_backend_tensor_view vx, vn, vo;
     gd_backend_matrix_view xm, wm, ym;
     gd_tensor last = f->h;
-    TRY(scratch(f->d->ctx, GD_DTYPE_F32, n, c->vocab, logits));
+    TRY(gd_decoder_logits(f->d, n, logits));
     if (!normed) {
         TRY(scratch(f->d->ctx, f->ll->type, n, c->width, &last));
         view2(&f->x, GD_BACKEND_DTYPE_F32, f->rows, c->width, &vx);

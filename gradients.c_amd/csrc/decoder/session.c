@@ -111,6 +111,7 @@ gd_status gd_gpt_decoder_step(gd_gpt_decoder *d, const int32_t *ids, int32_t *ne
     TRY(gd_begin_step(ctx, GD_SCOPE_INFER, gd_batch_empty()));
     st = data_i32(ctx, ids, d->cfg.batch, &t_ids);
     if (st == GD_OK) st = data_i32(ctx, d->pos, d->cfg.batch, &t_pos);
+    d->keep_logits = false;
     if (st == GD_OK) st = d->model->step(d, &t_ids, &t_pos, false, &t_logits);
     if (st == GD_OK) st = gd_argmax_rows(ctx, &t_logits, &t_next, &t_gaps);
     if (st != GD_OK) {
@@ -140,9 +141,10 @@ gd_status gd_gpt_decoder_prefill(gd_gpt_decoder *d, const int32_t *ids, const in
         if (cu[b + 1] <= cu[b] || cu[b + 1] - cu[b] > d->cfg.max_seq) return GD_ERR_INVALID_ARGUMENT;
     }
     TRY(gd_begin_step(ctx, GD_SCOPE_INFER, gd_batch_empty()));
+    /* the sampling front end starts from these logits without a round trip through the host */
+    d->keep_logits = true;
     st = d->model->prefill(d, ids, cu, &t_logits);
     if (st == GD_OK) st = gd_argmax_rows(ctx, &t_logits, &t_next, &t_gaps);
-    /* the sampling front end starts from these logits without a round trip through the host */
     if (st == GD_OK) st = keep_logits(d, &t_logits);
     if (st != GD_OK) {
         (void)gd_end_step(ctx);
@@ -218,6 +220,7 @@ gd_status gd_gpt_decoder_extend(gd_gpt_decoder *d, const int32_t *slots, int32_t
     st = gd_begin_step(d->ctx, GD_SCOPE_INFER, gd_batch_empty());
     if (st == GD_OK) {
         gd_status end;
+        d->keep_logits = false;
         st = d->model->extend(d, &e, &t_logits);
         end = gd_end_step(d->ctx);
         if (st == GD_OK) st = end;
@@ -272,9 +275,20 @@ static gd_status enqueue_sample(gd_gpt_decoder *d, const gd_tensor *logits, int3
     return gd_backend_sample_advance(gd_context_backend(d->ctx), &vl, &t, &a);
 }
 
-/* GD_GPT_RESIDENT_KEEP_LOGITS: the step's logits into the state tensor that outlives the step scope */
+gd_status gd_decoder_logits(gd_gpt_decoder *d, int64_t n, gd_tensor *logits)
+{
+    int64_t dims[2] = {n, d->cfg.vocab};
+    if (d->keep_logits && n == d->cfg.batch) {
+        *logits = d->last_logits;
+        return GD_OK;
+    }
+    return gd_tensor_empty(d->ctx, GD_ARENA_SCRATCH, d->last_logits.dtype, gd_shape_make(2U, dims), 256U, logits);
+}
+
+/* logits that a forward has not written there by itself, into the state tensor that outlives the step scope */
 static gd_status keep_logits(gd_gpt_decoder *d, const gd_tensor *logits)
 {
+    if (logits->storage.buffer == d->last_logits.storage.buffer && logits->storage.offset == d->last_logits.storage.offset) return GD_OK;
     return gd_backend_copy(gd_context_backend(d->ctx), (gd_backend_buffer *)d->last_logits.storage.buffer,
                            d->last_logits.storage.offset + d->last_logits.view_offset,
                            (gd_backend_buffer *)logits->storage.buffer, logits->storage.offset + logits->view_offset,
@@ -287,6 +301,7 @@ static gd_status enqueue_resident_step(gd_gpt_decoder *d)
     gd_tensor logits, next, gaps;
     gd_backend_tensor_view vl, vn, vg, vi, vp, vs, vo, vog, vt, vx;
     const int32_t delta = d->resident_hold ? 0 : 1;
+    d->keep_logits = d->resident_keep_logits != 0; /* GD_GPT_RESIDENT_KEEP_LOGITS */
     TRY(d->model->step(d, &d->ids_dev, &d->pos_dev, d->resident_unfused == 0, &logits));
     if (d->resident_sampling) return enqueue_sample(d, &logits, delta);
     if (d->resident_keep_logits) TRY(keep_logits(d, &logits));
