@@ -539,15 +539,43 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         }
         return h;
     };
+#if GD_LINEAR_IS_BF16
+    auto quad_gated = [&](auto mode_tag, const gd_float16 &value, const gd_float16 &gate, int j, int q) __attribute__((always_inline)) {
+        gd_elem4 h;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            float fv = value[4 * q + t], fg = gate[4 * q + t];
+            if (decltype(mode_tag)::value == GD_HIP_EPI_BIAS_F32) {
+                fv += (float)bq[j][q][t];
+                fg += (float)bq[j + WN / 2][q][t];
+            }
+            h[t] = (gd_elem)gd_tile_gated(fv, fg, p);
+        }
+        return h;
+    };
+#endif
     auto epilogue_pass = [&](auto pass_tag, auto mode_tag) __attribute__((always_inline)) {
         constexpr int I = decltype(pass_tag)::value;
         const uint32_t e = wm * 32u + frag_row;
+#if GD_LINEAR_IS_BF16
+        /* gated from the F32 sums, as in a whole tile: which tile a row lies in does not show in its bits */
+        constexpr int STAGED = WN / 2;
+#else
+        constexpr int STAGED = WN;
+#endif
 #pragma unroll
         for (int j = 0; j < WN; ++j) {
+            if (gated && j >= STAGED) break;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const uint32_t lc = wn * (WN * 32u) + (uint32_t)j * 32u + 8u * (uint32_t)q + 4u * frag_c;
-                *reinterpret_cast<gd_elem4 *>(epi + (e * EU + ((lc >> 2) ^ (e & 31u))) * 8u) = quad_f16(mode_tag, acc[I][j], j, q);
+                gd_elem4 h;
+#if GD_LINEAR_IS_BF16
+                if (gated && j < WN / 2) h = quad_gated(mode_tag, acc[I][j], acc[I][(j + WN / 2) % WN], j, q);
+                else
+#endif
+                h = quad_f16(mode_tag, acc[I][j], j, q);
+                *reinterpret_cast<gd_elem4 *>(epi + (e * EU + ((lc >> 2) ^ (e & 31u))) * 8u) = h;
             }
         }
         __syncthreads();
@@ -566,7 +594,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
             return h;
         };
         if (gated) {
-            /* a value chunk and the gate chunk HW/8 behind it make one output chunk */
+            /* a value chunk and the gate chunk HW/8 behind it make one output chunk (F16; BF16: multiplied already) */
 #pragma unroll
             for (uint32_t idx0 = 0; idx0 < 32u * CPRW; idx0 += 256u) {
                 const uint32_t idx = idx0 + tid;
@@ -575,10 +603,12 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 if (gr >= row_end || gc >= p.N) continue;
                 /* staged columns: wavefront column wc holds its HW value columns, then their gates */
                 const uint32_t cv = (v / (HW / 8u)) * (HW / 4u) + v % (HW / 8u);
-                const gd_elem8 hv = read_chunk(er, cv), hg = read_chunk(er, cv + HW / 8u);
-                gd_elem8 h;
+                gd_elem8 h = read_chunk(er, cv);
+#if !GD_LINEAR_IS_BF16
+                const gd_elem8 hg = read_chunk(er, cv + HW / 8u);
 #pragma unroll
-                for (int t = 0; t < 8; ++t) h[t] = (gd_elem)gd_tile_gated((float)hv[t], (float)hg[t], p);
+                for (int t = 0; t < 8; ++t) h[t] = (gd_elem)gd_tile_gated((float)h[t], (float)hg[t], p);
+#endif
                 gd_elem *yr = y + (size_t)gr * p.ldy + gc;
                 if (vector_store && gc + 8u <= p.N) {
                     *reinterpret_cast<gd_elem8 *>(yr) = h;
@@ -715,16 +745,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
 #pragma unroll
                     for (int s2 = 0; s2 < 2; ++s2) {
 #if GD_LINEAR_IS_BF16
-#pragma unroll
-                        for (int t = 0; t < 4; ++t) {
-                            const int q = 2 * pr + s2;
-                            float fv = acc[I][j][4 * q + t], fg = acc[I][j + WN / 2][4 * q + t];
-                            if (decltype(mode_tag)::value == GD_HIP_EPI_BIAS_F32) {
-                                fv += (float)bq[j][q][t];
-                                fg += (float)bq[j + WN / 2][q][t];
-                            }
-                            o[s2][t] = (gd_elem)gd_tile_gated(fv, fg, p);
-                        }
+                        o[s2] = quad_gated(mode_tag, acc[I][j], acc[I][j + WN / 2], j, 2 * pr + s2);
 #else
                         const gd_elem4 hv = quad_f16(mode_tag, acc[I][j], j, 2 * pr + s2);
                         const gd_elem4 hg = quad_f16(mode_tag, acc[I][j + WN / 2], j + WN / 2, 2 * pr + s2);

@@ -118,6 +118,20 @@ def test_big_tiles_and_unsupported_forms(backend, gda, arena):
     assert e.value.status == gda.UNSUPPORTED
 
 
+@pytest.mark.parametrize("kind", [1, 2])
+def test_a_gated_row_does_not_depend_on_its_tile(backend, gda, arena, kind):
+    """The rows of a last, ragged 256-row tile have the bits that the same rows have in a whole one."""
+    M, N, K = 300, 16640, 128
+    rng = np.random.default_rng(kind)
+    x, _ = _put(arena, BF16, rng.standard_normal((512, K)))
+    w, _ = _put(arena, BF16, rng.standard_normal((2 * N, K)) / np.sqrt(K))
+    b, _ = _put(arena, BF16, rng.standard_normal(2 * N))
+    whole, ragged = arena.alloc((512, N), BF16), arena.alloc((M, N), BF16)
+    backend.fused_linear(x, w, b, None, None, whole, True, 1, 0, epilogue=kind)
+    backend.fused_linear(x.rows(0, M), w, b, None, None, ragged, True, 1, 0, epilogue=kind)
+    assert np.array_equal(whole.read()[:M], ragged.read())
+
+
 # ---- residual stream --------------------------------------------------------------------------------------
 
 @TYPES
