@@ -3,9 +3,9 @@
  *   dt = softplus(dt_raw + dt_bias_h), S <- exp(-exp(a_log_h) dt) S + dt B x^T, y = S^T C + d_h x
  * with S [N, P] per head, in F32 from the first token to the last; B and C are shared by the heads of a group.
  *
- * One workgroup owns a [N, 32] column slice of one head of one sequence and keeps it in registers: thread (r, l) holds
- * rows r, r + 32, ... of columns 4l .. 4l+3, so a state row is read and written in whole 128-byte lines.  Tokens come
- * in batches of GD_SSM_BATCH through LDS; the column sums of S^T C go through wavefront shuffles and one LDS exchange
+ * One workgroup owns a [N, COLS] column slice of one head of one sequence and keeps it in registers: thread (r, l) holds
+ * rows r, r + R, ... (R = 1024 / COLS) of columns 4l .. 4l+3, so a state row is read and written in whole 128-byte lines.  Tokens come
+ * in batches through LDS; the column sums of S^T C go through wavefront shuffles and one LDS exchange
  * per batch.  This is the decode step (HBM-bound on reading and writing S once), the whole F32 path and the path of
  * short portions; long BF16 prompts take the matrix-core kernel of ssm_scan_chunk.hip.
  *
@@ -14,8 +14,6 @@
 #include "../../_shared/hip_device.h"
 #include "hip_ssm_scan_types.h"
 
-#define GD_SSM_BATCH 8
-#define GD_SSM_COLS 32
 #define GD_SSM_STATE_MAX 512
 
 __device__ __forceinline__ float gd_softplus(float v) { return fmaxf(v, 0.0f) + log1pf(expf(-fabsf(v))); }
@@ -49,27 +47,29 @@ __device__ __forceinline__ float gd_ssm_conv_at(const gd_hip_ssm_conv &cv, const
 /* CONV: xbc holds the inputs of the convolution (row pitch ld_xbc) and every sequence brings one token: the channels a
  * workgroup needs are convolved here.  B and C are convolved by every workgroup of their group; the places of the
  * ring that are read (positions in front of the token) and written (its own) differ, so they do not race. */
-template <typename T, int NR, bool CONV>
+template <typename T, int NR, bool CONV, int COLS = 32>
 __global__ void __launch_bounds__(256)
 gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, const float *__restrict__ dt_bias,
                    const float *__restrict__ a_log, const float *__restrict__ d_skip, float *__restrict__ states,
                    T *__restrict__ y, gd_hip_ssm_params m, gd_hip_ssm_conv cv, gd_hip_seqs q)
 {
-    __shared__ float sb[GD_SSM_BATCH][NR * 32], sc[GD_SSM_BATCH][NR * 32], sx[GD_SSM_BATCH][GD_SSM_COLS];
-    __shared__ float part[GD_SSM_BATCH][4][GD_SSM_COLS], sdt[GD_SSM_BATCH], sdec[GD_SSM_BATCH];
+    constexpr uint32_t GD_SSM_BATCH = CONV ? 1u : 8u, GD_SSM_COLS = COLS;
+    constexpr uint32_t L = GD_SSM_COLS / 4u, R = 256u / L, NS = NR * R; /* lanes of a row, rows of a pass, rows of all */
+    __shared__ __align__(16) float sb[GD_SSM_BATCH][NS], sc[GD_SSM_BATCH][NS], sx[GD_SSM_BATCH][GD_SSM_COLS];
+    __shared__ __align__(16) float part[GD_SSM_BATCH][4][GD_SSM_COLS], sdt[GD_SSM_BATCH], sdec[GD_SSM_BATCH];
     const uint32_t p0 = blockIdx.x * GD_SSM_COLS, h = blockIdx.y;
-    const uint32_t l = threadIdx.x & 7u, r = threadIdx.x >> 3, wave = threadIdx.x >> 6;
+    const uint32_t l = threadIdx.x % L, r = threadIdx.x / L, wave = threadIdx.x >> 6;
     const uint32_t N = m.state, P = m.vdim, inner = m.heads * P, g = h / (m.heads / m.groups);
     int32_t first, n, start, slot;
     if (!gd_seq_span(q, blockIdx.z, &first, &n, &start, &slot)) return;
     float *st = states + ((size_t)slot * m.heads + h) * N * P + p0;
     const float rate = expf(a_log[h]), bias = dt_bias[h], skip = d_skip[h];
-    const uint32_t cols = min(P - p0, (uint32_t)GD_SSM_COLS);
+    const uint32_t cols = min(P - p0, GD_SSM_COLS);
     const bool vec = (P & 3u) == 0u;
     gd_float4 S[NR];
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-        const uint32_t row = r + 32u * i;
+        const uint32_t row = r + R * i;
         S[i] = (gd_float4){0.f, 0.f, 0.f, 0.f};
         if (start > 0 && row < N && 4u * l < cols) {
             if (vec) S[i] = *reinterpret_cast<const gd_float4 *>(st + (size_t)row * P + 4u * l);
@@ -78,24 +78,24 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
         }
     }
     for (int32_t t0 = 0; t0 < n; t0 += GD_SSM_BATCH) {
-        const uint32_t nb = min((uint32_t)(n - t0), (uint32_t)GD_SSM_BATCH);
+        const uint32_t nb = min((uint32_t)(n - t0), GD_SSM_BATCH);
         const T *rows = xbc + (size_t)(first + t0) * m.ld_xbc;
         if (CONV) {
             T *rg = (T *)cv.ring + (size_t)slot * cv.K * cv.C;
             const bool own = blockIdx.x == 0u && h % (m.heads / m.groups) == 0u; /* of B and C of the group */
-            for (uint32_t i = threadIdx.x; i < 2u * NR * 32u + GD_SSM_COLS; i += 256u) {
-                const uint32_t k = i % (NR * 32u), part = i / (NR * 32u);
+            for (uint32_t i = threadIdx.x; i < 2u * NS + GD_SSM_COLS; i += 256u) {
+                const uint32_t k = i % (NS), part = i / (NS);
                 if (part < 2u) {
                     float *dst = part == 0u ? &sb[0][k] : &sc[0][k];
                     *dst = k < N ? gd_ssm_conv_at<T>(cv, rows, rg, inner + (part * m.groups + g) * N + k, start, own) : 0.f;
                 } else {
-                    const uint32_t c = i - 2u * NR * 32u;
+                    const uint32_t c = i - 2u * NS;
                     sx[0][c] = c < cols ? gd_ssm_conv_at<T>(cv, rows, rg, h * P + p0 + c, start, true) : 0.f;
                 }
             }
         } else {
-        for (uint32_t i = threadIdx.x; i < nb * (NR * 32u); i += 256u) {
-            const uint32_t t = i / (NR * 32u), k = i % (NR * 32u);
+        for (uint32_t i = threadIdx.x; i < nb * (NS); i += 256u) {
+            const uint32_t t = i / (NS), k = i % (NS);
             const T *b = rows + (size_t)t * m.ld_xbc + inner + g * N;
             sb[t][k] = k < N ? (float)b[k] : 0.f;
             sc[t][k] = k < N ? (float)b[m.groups * N + k] : 0.f;
@@ -117,7 +117,7 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
             gd_float4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
-                const float b = dt * sb[t][r + 32u * i], c = sc[t][r + 32u * i];
+                const float b = dt * sb[t][r + R * i], c = sc[t][r + R * i];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     S[i][e] = fmaf(dec, S[i][e], b * x4[e]);
@@ -126,11 +126,11 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
             }
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                acc[e] += __shfl_xor(acc[e], 8, 64);
+                if (L <= 8u) acc[e] += __shfl_xor(acc[e], 8, 64);
                 acc[e] += __shfl_xor(acc[e], 16, 64);
                 acc[e] += __shfl_xor(acc[e], 32, 64);
             }
-            if ((threadIdx.x & 63u) < 8u) *reinterpret_cast<gd_float4 *>(&part[t][wave][4u * l]) = acc;
+            if ((threadIdx.x & 63u) < L) *reinterpret_cast<gd_float4 *>(&part[t][wave][4u * l]) = acc;
         }
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < nb * GD_SSM_COLS; i += 256u) {
@@ -143,7 +143,7 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
     }
 #pragma unroll
     for (int i = 0; i < NR; ++i) {
-        const uint32_t row = r + 32u * i;
+        const uint32_t row = r + R * i;
         if (row < N && 4u * l < cols) {
             if (vec) *reinterpret_cast<gd_float4 *>(st + (size_t)row * P + 4u * l) = S[i];
             else
@@ -157,7 +157,11 @@ extern "C" int gd_hip_launch_ssm_scan(hipStream_t stream, const void *xbc, const
                                       const gd_hip_ssm_params *m, const gd_hip_ssm_conv *cv, const gd_hip_seqs *q,
                                       int is_f32)
 {
-    const dim3 grid((m->vdim + GD_SSM_COLS - 1u) / GD_SSM_COLS, m->heads, q->seqs);
+    /* a decode step over whole 64-column slices: half as many workgroups convolve the B and C of their group once more, and each has
+     * twice the state on its way (64 sequences x 32 heads of [128, 64]: 38.4 -> 32.1 us, 4.2 TB/s of state) */
+    const bool pair = cv != nullptr && (m->vdim % 64u) == 0u && m->state <= 256u;
+    const uint32_t slice = pair ? 64u : 32u;
+    const dim3 grid((m->vdim + slice - 1u) / slice, m->heads, q->seqs);
     if (q->rows == 0u || q->seqs == 0u) return (int)hipSuccess;
     if (m->state > GD_SSM_STATE_MAX) return (int)hipErrorInvalidValue;
     const gd_hip_ssm_conv none = {nullptr, nullptr, nullptr, 0u, 0u};
@@ -170,11 +174,21 @@ extern "C" int gd_hip_launch_ssm_scan(hipStream_t stream, const void *xbc, const
         else if (m->state <= 256u) GD_GO(T, 8, CONV); \
         else GD_GO(T, 16, CONV);                      \
     } while (0)
-    if (cv != nullptr) {
+#define GD_PAIR(T)                                                                                                                  \
+    do {                                                                                                                            \
+        const T *xt = (const T *)xbc, *dt = (const T *)dt_raw;                                                                      \
+        if (m->state <= 64u) gd_ssm_scan_kernel<T, 4, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q);       \
+        else if (m->state <= 128u) gd_ssm_scan_kernel<T, 8, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q); \
+        else gd_ssm_scan_kernel<T, 16, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q);                      \
+    } while (0)
+    if (pair) {
+        if (is_f32) GD_PAIR(float); else GD_PAIR(gd_bf16);
+    } else if (cv != nullptr) {
         if (is_f32) GD_PICK(float, true); else GD_PICK(gd_bf16, true);
     } else {
         if (is_f32) GD_PICK(float, false); else GD_PICK(gd_bf16, false);
     }
+#undef GD_PAIR
 #undef GD_PICK
 #undef GD_GO
     return (int)hipGetLastError();

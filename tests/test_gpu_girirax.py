@@ -302,6 +302,12 @@ def test_fused_convolution_and_recurrence_step(backend, gda, arena, dtype, H, P,
 
 
 @TYPES
+@pytest.mark.parametrize("H,P,N,Gn,K", [(2, 64, 33, 1, 4), (3, 128, 128, 3, 2), (1, 192, 200, 1, 4), (4, 64, 256, 2, 5)])
+def test_fused_step_over_64_column_slices(backend, gda, arena, dtype, H, P, N, Gn, K):
+    test_fused_convolution_and_recurrence_step(backend, gda, arena, dtype, H, P, N, Gn, K)
+
+
+@TYPES
 @pytest.mark.parametrize("inner,parts", [(64, 1), (96, 4), (4096, 2), (30, 3), (5000, 1)])
 def test_gate_then_group_norm(backend, gda, arena, L, dtype, inner, parts):
     rng = np.random.default_rng(inner)
