@@ -12,6 +12,7 @@
 
 #define GD_RN_THREADS 256
 #define GD_RN_CHUNKS 4 /* 8-element chunks per thread on the register path */
+#define GD_RN_PLACES 2u /* choices of a row whose places are requested ahead */
 
 template <typename T>
 struct gd_rn_vec;
@@ -89,19 +90,22 @@ gd_residual_embed_kernel(const T *__restrict__ table, const int32_t *__restrict_
     }
 }
 
-template <typename T, bool VEC>
+/* LANES as in gd_residual_add_norm_kernel */
+template <typename T, bool VEC, int LANES>
 __global__ void __launch_bounds__(GD_RN_THREADS)
 gd_residual_norm_add_kernel(const T *__restrict__ u, const float *__restrict__ w, float *__restrict__ x,
-                            T *__restrict__ copy, uint32_t cols, float eps, float mult)
+                            T *__restrict__ copy, uint32_t cols, float eps, float mult, uint32_t n_rows)
 {
     __shared__ float red[GD_RN_THREADS / 64];
-    const size_t base = (size_t)blockIdx.x * cols;
+    const uint32_t row = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES, sub = threadIdx.x % LANES;
+    if (LANES < GD_RN_THREADS && row >= n_rows) return;
+    const size_t base = (size_t)row * cols;
     float ss = 0.f;
     if (VEC) {
         float uv[GD_RN_CHUNKS][8], xv[GD_RN_CHUNKS][8], wv[GD_RN_CHUNKS][8]; /* all requested in front of the sum */
 #pragma unroll
         for (int i = 0; i < GD_RN_CHUNKS; ++i) {
-            const uint32_t c = (threadIdx.x + i * GD_RN_THREADS) * 8u;
+            const uint32_t c = (sub + i * LANES) * 8u;
             if (c >= cols) continue;
             gd_rn_vec<T>::load(u + base + c, uv[i]);
             gd_rn_vec<float>::load(x + base + c, xv[i]);
@@ -109,15 +113,15 @@ gd_residual_norm_add_kernel(const T *__restrict__ u, const float *__restrict__ w
         }
 #pragma unroll
         for (int i = 0; i < GD_RN_CHUNKS; ++i) {
-            if ((threadIdx.x + i * GD_RN_THREADS) * 8u >= cols) continue;
+            if ((sub + i * LANES) * 8u >= cols) continue;
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss = fmaf(uv[i][e], uv[i][e], ss);
         }
-        ss = gd_block_sum<GD_RN_THREADS / 64>(ss, red);
+        ss = LANES == 64 ? gd_wave_sum(ss) : gd_block_sum<GD_RN_THREADS / 64>(ss, red);
         const float inv = 1.0f / sqrtf(ss / (float)cols + eps);
 #pragma unroll
         for (int i = 0; i < GD_RN_CHUNKS; ++i) {
-            const uint32_t c = (threadIdx.x + i * GD_RN_THREADS) * 8u;
+            const uint32_t c = (sub + i * LANES) * 8u;
             if (c >= cols) continue;
 #pragma unroll
             for (int e = 0; e < 8; ++e) xv[i][e] += mult * (uv[i][e] * inv * wv[i][e]);
@@ -140,8 +144,9 @@ gd_residual_norm_add_kernel(const T *__restrict__ u, const float *__restrict__ w
 }
 
 /* u, w and out may be null; choices of a row: rows place[row * top + k] of the packed rows, negative: none.  LANES
- * threads per row, 256 or 64 (a wavefront: no exchange through LDS, for many short rows).  VEC: rows of up to 8 * LANES * 4
- * elements in 16-byte pieces, in registers between the sum of squares and the stores. */
+ * threads per row, 256 or 64 (a wavefront: no exchange through LDS, for short rows).  VEC: rows of up to 8 * LANES * 4
+ * elements in 16-byte pieces, in registers between the sum of squares and the stores; the places of a row's first choices are
+ * requested with them, so that the choices' rows are one dependent round trip away and not two. */
 template <typename T, bool VEC, int LANES>
 __global__ void __launch_bounds__(GD_RN_THREADS)
 gd_residual_add_norm_kernel(const T *__restrict__ u, gd_hip_routed_choice<T> in, float *__restrict__ x,
@@ -149,11 +154,17 @@ gd_residual_add_norm_kernel(const T *__restrict__ u, gd_hip_routed_choice<T> in,
                             float eps, uint32_t n_rows)
 {
     __shared__ float red[GD_RN_THREADS / 64];
-    const uint32_t row = blockIdx.x * (GD_RN_THREADS / LANES) + threadIdx.x / LANES, sub = threadIdx.x % LANES;
+    const uint32_t row = blockIdx.x * (blockDim.x / LANES) + threadIdx.x / LANES, sub = threadIdx.x % LANES;
     if (LANES < GD_RN_THREADS && row >= n_rows) return;
     const size_t base = (size_t)row * cols;
     float ss = 0.f;
     if (VEC) {
+        int32_t from[GD_RN_PLACES], onto[GD_RN_PLACES];
+#pragma unroll
+        for (uint32_t k = 0; k < GD_RN_PLACES; ++k) {
+            from[k] = k < in.top ? in.place[row * in.top + k] : -1;
+            onto[k] = k < to.top ? to.place[row * to.top + k] : -1;
+        }
         float uv[GD_RN_CHUNKS][8], xv[GD_RN_CHUNKS][8], wv[GD_RN_CHUNKS][8]; /* all requested in front of the sums */
 #pragma unroll
         for (int i = 0; i < GD_RN_CHUNKS; ++i) {
@@ -172,7 +183,7 @@ gd_residual_add_norm_kernel(const T *__restrict__ u, gd_hip_routed_choice<T> in,
             }
         }
         for (uint32_t k = 0; k < in.top; ++k) {
-            const int32_t at = in.place[row * in.top + k];
+            const int32_t at = k < GD_RN_PLACES ? (k == 0u ? from[0] : from[1]) : in.place[row * in.top + k];
             if (at < 0 || (uint32_t)at >= in.rows) continue;
 #pragma unroll
             for (int i = 0; i < GD_RN_CHUNKS; ++i) {
@@ -207,7 +218,7 @@ gd_residual_add_norm_kernel(const T *__restrict__ u, gd_hip_routed_choice<T> in,
             gd_rn_vec<T>::store(out + base + c, xv[i]);
         }
         for (uint32_t k = 0; k < to.top; ++k) {
-            const int32_t at = to.place[row * to.top + k];
+            const int32_t at = k < GD_RN_PLACES ? (k == 0u ? onto[0] : onto[1]) : to.place[row * to.top + k];
             if (at < 0 || (uint32_t)at >= to.rows) continue;
 #pragma unroll
             for (int i = 0; i < GD_RN_CHUNKS; ++i) {
@@ -268,15 +279,32 @@ extern "C" int gd_hip_launch_residual_embed(hipStream_t stream, const void *tabl
     return (int)hipGetLastError();
 }
 
+/* A wavefront per row up to 1024 columns, where a workgroup would leave half of its threads idle: four rows to a workgroup where
+ * there are many (40,796 rows: 155 -> 101 us), one where there are few, so that they spread over the compute units (64 rows of a
+ * decode step: 5.2 -> 4.8 us).  At 2048 columns a workgroup per row is as fast (16 rows: 6.3 against 6.4 us). */
+struct gd_rn_shape {
+    bool wave;
+    uint32_t threads, groups;
+};
+static gd_rn_shape gd_rn_shape_of(bool vec, uint32_t rows, uint32_t cols)
+{
+    if (!vec || cols > 1024u) return {false, GD_RN_THREADS, rows};
+    if (rows >= 1024u) return {true, GD_RN_THREADS, (rows + GD_RN_THREADS / 64u - 1u) / (GD_RN_THREADS / 64u)};
+    return {true, 64u, rows};
+}
+
 extern "C" int gd_hip_launch_residual_norm_add(hipStream_t stream, const void *u, const float *w, float *x, void *copy,
                                                uint32_t rows, uint32_t cols, float eps, float mult, int is_f32,
                                                int aligned16)
 {
     if (rows == 0u) return (int)hipSuccess;
     const bool vec = aligned16 && (cols % 8u) == 0u && cols <= 8u * GD_RN_THREADS * GD_RN_CHUNKS;
-#define GD_GO(T, V) gd_residual_norm_add_kernel<T, V><<<rows, GD_RN_THREADS, 0, stream>>>((const T *)u, w, x, (T *)copy, cols, eps, mult)
-    if (is_f32) { if (vec) GD_GO(float, true); else GD_GO(float, false); }
-    else { if (vec) GD_GO(gd_bf16, true); else GD_GO(gd_bf16, false); }
+    const gd_rn_shape shape = gd_rn_shape_of(vec, rows, cols);
+#define GD_GO(T, V, L) gd_residual_norm_add_kernel<T, V, L><<<shape.groups, shape.threads, 0, stream>>>((const T *)u, w, x, (T *)copy, cols, eps, mult, rows)
+#define GD_GO_TYPE(T) do { if (shape.wave) GD_GO(T, true, 64); else if (vec) GD_GO(T, true, 256); else GD_GO(T, false, 256); } while (0)
+    if (is_f32) GD_GO_TYPE(float);
+    else GD_GO_TYPE(gd_bf16);
+#undef GD_GO_TYPE
 #undef GD_GO
     return (int)hipGetLastError();
 }
@@ -289,14 +317,12 @@ extern "C" int gd_hip_launch_residual_add_norm(hipStream_t stream, const void *u
 {
     if (rows == 0u) return (int)hipSuccess;
     const bool vec = aligned16 && (cols % 8u) == 0u && cols <= 8u * GD_RN_THREADS * GD_RN_CHUNKS;
-    /* a wavefront per row where a workgroup would leave half of its threads idle and there are rows enough (1024 columns,
-     * 40,796 rows: 155 -> 101 us; at 2048 columns a workgroup is as fast) */
-    const bool wave = vec && cols <= 1024u && rows >= 1024u;
+    const gd_rn_shape shape = gd_rn_shape_of(vec, rows, cols);
 #define GD_GO(T, V, L)                                                                                                 \
-    gd_residual_add_norm_kernel<T, V, L><<<(rows + GD_RN_THREADS / L - 1u) / (GD_RN_THREADS / L), GD_RN_THREADS, 0, stream>>>( \
+    gd_residual_add_norm_kernel<T, V, L><<<shape.groups, shape.threads, 0, stream>>>(                                  \
         (const T *)u, gd_hip_routed_choice<T>{(T *)in, in_place, in_rows, in_top, in_weight}, x, w, (T *)out,          \
         gd_hip_routed_choice<T>{(T *)to, to_place, to_rows, to_top, 1.0f}, cols, eps, rows)
-#define GD_GO_TYPE(T) do { if (wave) GD_GO(T, true, 64); else if (vec) GD_GO(T, true, 256); else GD_GO(T, false, 256); } while (0)
+#define GD_GO_TYPE(T) do { if (shape.wave) GD_GO(T, true, 64); else if (vec) GD_GO(T, true, 256); else GD_GO(T, false, 256); } while (0)
     if (is_f32) GD_GO_TYPE(float);
     else GD_GO_TYPE(gd_bf16);
 #undef GD_GO_TYPE
