@@ -143,6 +143,11 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
             const uint32_t qpw = (p.K / 128u + 7u) / 8u; /* pieces of 128 per wavefront */
             if (qpw <= 2u) { launch_wide_half<2>(stream, x, w, bias, residual, y, p); return 1; }
             if (qpw <= 6u) { launch_wide_half<6>(stream, x, w, bias, residual, y, p); return 1; }
+#if GD_LINEAR_IS_BF16
+            /* (8448 -> 2048 at 4 and 16 rows: 12.7 and 17.0 us, the stream kernel's four wavefronts 14.7 and 18.3; what is left is the
+             * activation matrix, which every 8 columns read whole) */
+            if (qpw <= 12u) { launch_wide_half<12>(stream, x, w, bias, residual, y, p); return 1; }
+#endif
         }
         if (ppw <= 4u) GD_W(1, 1, 4, GD_HIP_PRO_NONE, GD_WIDE_EPI_PLAIN);
         if (ppw <= 12u) GD_W(1, 1, 12, GD_HIP_PRO_NONE, GD_WIDE_EPI_PLAIN);
