@@ -882,6 +882,34 @@ def test_argmax_rows(backend, arena, oracle, gda):
     assert np.array_equal(ids2.read(), oracle.argmax_rows(wide)[0])
 
 
+@pytest.mark.parametrize("half", [True, False])
+@pytest.mark.parametrize("cols", [1, 7, 260, 8191, 8192, 32768, 32772, 70001])
+def test_argmax_rows_ends_of_the_scan(backend, arena, oracle, gda, cols, half):
+    """largest finite value, lowest index among equals, distance to the runner-up: rows with the leader at either end, equal
+    leaders, infinities and NaN, one finite value, none.  Exact: values are compared, not computed."""
+    dtype = np.float16 if half else np.float32
+    x = oracle.normal_f16((9, cols), 1602 + cols, 3.0).astype(dtype)
+    top = dtype(40.0)
+    x[1, 0] = x[2, -1] = top
+    x[3, [0, cols // 2, -1]] = top
+    x[4, ::3], x[4, 1::3] = np.inf, np.nan
+    x[5, ::2], x[5, -1] = -np.inf, np.finfo(dtype).min
+    x[6], x[6, cols // 3] = np.nan, dtype(-2.0)
+    x[7], x[8] = -np.inf, np.finfo(dtype).tiny * np.sign(np.arange(cols) - cols // 2)
+    ids, gap = arena.alloc((9,), gda.I32), arena.alloc((9,), gda.F32)
+    backend.argmax_rows(arena.from_numpy(x), ids, gap)
+    v = np.where(np.isfinite(x), x, -np.inf).astype(np.float32)
+    best = v.argmax(1)  # the first of equals
+    lead = v[np.arange(9), best]
+    rest = v.copy()
+    rest[np.arange(9), best] = -np.inf
+    second = rest.max(1)
+    want = np.full(9, np.inf, np.float32)
+    np.subtract(lead, second, out=want, where=np.isfinite(second))
+    assert np.array_equal(ids.read(), np.where(np.isfinite(lead), best, 0))
+    assert np.array_equal(gap.read(), want)
+
+
 def test_gather_rows_and_position_increment(backend, arena, oracle, gda):
     src = oracle.normal_f16((100, 512), 1700)
     rows = np.array([99, 0, 42, 42, 100], np.int32)  # last one is out of range: row untouched
