@@ -5,7 +5,7 @@
  *   absorb  q_lat[h] = W_uk[h]^T q[h] per 16 rows, head and 64 latent columns, and the rotated query part behind it
  *   attend  a workgroup of 4 wavefronts takes 16 or 32 heads of one token over a piece of its keys: a cache row is read from
  *           memory once for all of them.  HBM-bound on the cache rows.
- *   merge   the pieces of a token and head into one latent vector
+ *   merge   the pieces of a token and head into one latent vector (where there are few, a part of value)
  *   value   16 tokens and one head: the value up-projection and the output gate
  *
  * attend.  Keys advance in tiles of 32 rows through two LDS stages filled by global -> LDS loads; two workgroups share a
@@ -31,28 +31,37 @@
 
 #define GD_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0)
 #define GD_LD_TILE 32u
+/* pieces up to which the value kernel merges them itself: one launch less, while each of its ceil(vdim / 32) workgroups per head
+ * reads the pieces again (64 rows, 8 heads, vdim 128, kv_rank 256: 7.3 us against 5.0 + 4.8); more pieces come with few rows,
+ * where the merge kernel spreads their latents over more wavefronts */
+#define GD_LD_FOLD 8u
 
-/* grid (ceil(kv_rank / 64), heads, ceil(rows / 16)); dim % 8 == 0, rot_dim % 8 == 0 (16-byte fragments of q) */
+/* grid (ceil(kv_rank / 64) + 1, heads, ceil(rows / 16)); dim % 8 == 0, rot_dim % 8 == 0 (16-byte fragments of q).  A chain of round
+ * trips, so the fragments of four steps are requested together and the rotated part has a workgroup of its own, the last of x
+ * (64 rows, 8 heads, dim 128, kv_rank 256: 5.6 -> 4.1 us) */
 __global__ void __launch_bounds__(256)
 gd_latent_absorb_kernel(const gd_bf16 *__restrict__ qv, const gd_bf16 *__restrict__ w_ukt,
                         const float *__restrict__ angles, gd_bf16 *__restrict__ ql, gd_hip_latent_params m, uint32_t rows)
 {
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, li = lane & 15u, lg = lane >> 4;
     const uint32_t h = blockIdx.y, r0 = blockIdx.z * 16u, hd = m.dim + m.rot_dim;
-    const uint32_t c0 = blockIdx.x * 64u + wave * 16u;
-    const gd_bf16 *qr = qv + ((size_t)min(r0 + li, rows - 1u) * m.heads + h) * hd;
-    if (c0 < m.kv_rank) {
+    if (blockIdx.x + 1u < gridDim.x) {
+        const uint32_t c0 = blockIdx.x * 64u + wave * 16u;
+        if (c0 >= m.kv_rank) return;
+        const gd_bf16 *qr = qv + ((size_t)min(r0 + li, rows - 1u) * m.heads + h) * hd;
         const gd_bf16 *wr = w_ukt + ((size_t)h * m.kv_rank + min(c0 + li, m.kv_rank - 1u)) * m.dim;
         const gd_bf16x8 zero = (gd_bf16x8)(gd_bf16)0.f;
         gd_float4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (uint32_t k = 0; k < m.dim; k += 32u) {
-            const uint32_t kk = k + 8u * lg;
-            gd_bf16x8 a = zero, b = zero;
-            if (kk < m.dim) {
-                a = *reinterpret_cast<const gd_bf16x8 *>(qr + kk);
-                b = *reinterpret_cast<const gd_bf16x8 *>(wr + kk);
+        for (uint32_t k = 0; k < m.dim; k += 128u) {
+            gd_bf16x8 a[4], b[4];
+#pragma unroll
+            for (uint32_t t = 0; t < 4u; ++t) {
+                const uint32_t kk = k + 32u * t + 8u * lg;
+                a[t] = kk < m.dim ? *reinterpret_cast<const gd_bf16x8 *>(qr + kk) : zero;
+                b[t] = kk < m.dim ? *reinterpret_cast<const gd_bf16x8 *>(wr + kk) : zero;
             }
-            acc = GD_MFMA(a, b, acc);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc = GD_MFMA(a[t], b[t], acc);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -60,8 +69,8 @@ gd_latent_absorb_kernel(const gd_bf16 *__restrict__ qv, const gd_bf16 *__restric
             if (row < rows && c0 + li < m.kv_rank)
                 ql[((size_t)row * m.heads + h) * m.pitch + c0 + li] = (gd_bf16)acc[r];
         }
+        return;
     }
-    if (blockIdx.x != 0u) return;
     const uint32_t half = m.rot_dim / 2u, tail = m.pitch - m.kv_rank;
     for (uint32_t i = threadIdx.x; i < 16u * tail; i += 256u) {
         const uint32_t row = r0 + i / tail, e = i % tail;
@@ -309,25 +318,55 @@ gd_latent_merge_kernel(const float *__restrict__ o_part, const float *__restrict
     }
 }
 
-/* grid (ceil(vdim / 32), heads, ceil(rows / 16)); kv_rank % 16 == 0 */
+/* grid (ceil(vdim / 32), heads, ceil(rows / 16)); kv_rank % 16 == 0.  PIECES: the pieces of a token and head (at most
+ * GD_LD_FOLD) are merged here, as gd_latent_merge_kernel merges them, by every workgroup that needs them */
+template <bool PIECES>
 __global__ void __launch_bounds__(256)
-gd_latent_value_mfma_kernel(const gd_bf16 *__restrict__ merged, const gd_bf16 *__restrict__ w_uv,
+gd_latent_value_mfma_kernel(const gd_bf16 *__restrict__ merged, const float *__restrict__ o_part,
+                            const float *__restrict__ ml, const gd_bf16 *__restrict__ w_uv,
                             const gd_bf16 *__restrict__ gate, uint32_t ldg, gd_bf16 *__restrict__ out,
-                            gd_hip_latent_params m, uint32_t rows)
+                            gd_hip_latent_params m, gd_hip_seqs q)
 {
     __shared__ float s_acc[2][64][4];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, li = lane & 15u, lg = lane >> 4;
-    const uint32_t h = blockIdx.y, r0 = blockIdx.z * 16u;
+    const uint32_t h = blockIdx.y, r0 = blockIdx.z * 16u, rows = q.rows, own = min(r0 + li, rows - 1u);
     /* wavefront: column tile wave % 2, half wave / 2 of the latent columns */
     const uint32_t v0 = blockIdx.x * 32u + (wave & 1u) * 16u, steps = (m.kv_rank + 31u) / 32u;
     const uint32_t s_begin = (wave >> 1) * ((steps + 1u) / 2u), s_end = (wave >> 1) ? steps : (steps + 1u) / 2u;
     const gd_bf16 *wr = w_uv + ((size_t)h * m.vdim + min(v0 + li, m.vdim - 1u)) * m.kv_rank;
-    const gd_bf16 *mr = merged + ((size_t)min(r0 + li, rows - 1u) * m.heads + h) * m.kv_rank;
+    const gd_bf16 *mr = merged + ((size_t)own * m.heads + h) * m.kv_rank;
+    const float *pr = o_part + ((size_t)own * m.pieces * m.heads + h) * m.kv_rank;
     const gd_bf16x8 zero = (gd_bf16x8)(gd_bf16)0.f;
     float g[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         g[r] = (float)gate[(size_t)min(r0 + 4u * lg + (uint32_t)r, rows - 1u) * ldg + h * m.vdim + min(v0 + li, m.vdim - 1u)];
+    /* PIECES: lane group lg holds the weights of pieces lg and 4 + lg of its lane's row */
+    uint32_t live = 0u;
+    float weight[2] = {0.f, 0.f};
+    if (PIECES) {
+        int32_t seq, pos, slot;
+        if (gd_seq_of_row(q, own, &seq, &pos, &slot))
+            live = min((min((uint32_t)pos + 1u, m.tmax) + m.piece_keys - 1u) / m.piece_keys, m.pieces);
+        float ref[2], part[2];
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) {
+            const bool has = 4u * i + lg < live;
+            const float *v = ml + (((size_t)own * m.pieces + (has ? 4u * i + lg : 0u)) * m.heads + h) * 2u;
+            ref[i] = has ? v[0] : -INFINITY;
+            part[i] = has ? v[1] : 0.f;
+        }
+        float top = fmaxf(ref[0], ref[1]);
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+#pragma unroll
+        for (uint32_t i = 0; i < 2u; ++i) weight[i] = 4u * i + lg < live ? __builtin_amdgcn_exp2f(ref[i] - top) : 0.f;
+        float total = weight[0] * part[0] + weight[1] * part[1];
+        total += __shfl_xor(total, 32, 64);
+        total += __shfl_xor(total, 16, 64);
+        weight[0] /= total;
+        weight[1] /= total;
+    }
     gd_float4 acc = {0.f, 0.f, 0.f, 0.f};
     for (uint32_t s = s_begin; s < s_end; s += 4u) { /* the loads of four steps together */
         gd_bf16x8 a[4], b[4];
@@ -335,8 +374,42 @@ gd_latent_value_mfma_kernel(const gd_bf16 *__restrict__ merged, const gd_bf16 *_
         for (uint32_t t = 0; t < 4u; ++t) {
             const uint32_t c = 32u * (s + t) + 8u * lg;
             const bool ok = s + t < s_end && c < m.kv_rank;
-            a[t] = ok ? *reinterpret_cast<const gd_bf16x8 *>(mr + c) : zero;
+            if (!PIECES) a[t] = ok ? *reinterpret_cast<const gd_bf16x8 *>(mr + c) : zero;
             b[t] = ok ? *reinterpret_cast<const gd_bf16x8 *>(wr + c) : zero;
+        }
+        if (PIECES) {
+            float sum[2][4][8]; /* of the even and of the odd pieces */
+#pragma unroll
+            for (int i = 0; i < 64; ++i) sum[i >> 5][(i >> 3) & 3][i & 7] = 0.f;
+            for (uint32_t p = 0; p < m.pieces; p += 2u) {
+                if (__ballot(p < live) == 0ull) break;
+                gd_float4 v[2][4][2];
+#pragma unroll
+                for (uint32_t i = 0; i < 2u; ++i)
+#pragma unroll
+                    for (uint32_t t = 0; t < 4u; ++t) {
+                        const uint32_t c = 32u * (s + t) + 8u * lg;
+                        const bool ok = p + i < live && s + t < s_end && c < m.kv_rank;
+                        const float *src = pr + (size_t)(ok ? p + i : 0u) * m.heads * m.kv_rank + (ok ? c : 0u);
+#pragma unroll
+                        for (int e = 0; e < 2; ++e)
+                            v[i][t][e] = ok ? reinterpret_cast<const gd_float4 *>(src)[e] : (gd_float4){0.f, 0.f, 0.f, 0.f};
+                    }
+#pragma unroll
+                for (uint32_t i = 0; i < 2u; ++i) {
+                    const uint32_t from = li + 16u * ((p + i) & 3u);
+                    const float w0 = __shfl(weight[0], (int)from, 64), w1 = __shfl(weight[1], (int)from, 64);
+                    const float w = p + i < live ? (p + i < 4u ? w0 : w1) : 0.f;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) sum[i][t][e] = fmaf(w, v[i][t][e >> 2][e & 3], sum[i][t][e]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[t][e] = (gd_bf16)(sum[0][t][e] + sum[1][t][e]);
         }
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc = GD_MFMA(a[t], b[t], acc);
@@ -380,7 +453,7 @@ extern "C" int gd_hip_launch_latent_decode(hipStream_t stream, const void *qv, c
     const uint32_t steps = (m.pitch + 31u) / 32u, rt = (q.rows + 15u) / 16u;
     const gd_bf16 *qlp = (const gd_bf16 *)ql, *cp = (const gd_bf16 *)cache;
     int e;
-    gd_latent_absorb_kernel<<<dim3((m.kv_rank + 63u) / 64u, m.heads, rt), 256, 0, stream>>>(
+    gd_latent_absorb_kernel<<<dim3((m.kv_rank + 63u) / 64u + 1u, m.heads, rt), 256, 0, stream>>>(
         (const gd_bf16 *)qv, (const gd_bf16 *)w_ukt, angles, (gd_bf16 *)ql, m, q.rows);
     e = (int)hipGetLastError();
     if (e != 0) return e;
@@ -392,11 +465,17 @@ extern "C" int gd_hip_launch_latent_decode(hipStream_t stream, const void *qv, c
     else return (int)hipErrorInvalidValue;
 #undef GD_GO
     if (e != 0) return e;
+    const dim3 values((m.vdim + 31u) / 32u, m.heads, rt);
+    if (m.pieces <= GD_LD_FOLD) {
+        gd_latent_value_mfma_kernel<true><<<values, 256, 0, stream>>>(
+            nullptr, o_part, ml, (const gd_bf16 *)w_uv, (const gd_bf16 *)gate, ldg, (gd_bf16 *)out, m, q);
+        return (int)hipGetLastError();
+    }
     /* the queries are used up: their place takes the merged latents (kv_rank <= pitch) */
     gd_latent_merge_kernel<<<dim3(q.rows, m.heads), 256, 0, stream>>>(o_part, ml, (gd_bf16 *)ql, m, q);
     e = (int)hipGetLastError();
     if (e != 0) return e;
-    gd_latent_value_mfma_kernel<<<dim3((m.vdim + 31u) / 32u, m.heads, rt), 256, 0, stream>>>(
-        qlp, (const gd_bf16 *)w_uv, (const gd_bf16 *)gate, ldg, (gd_bf16 *)out, m, q.rows);
+    gd_latent_value_mfma_kernel<false><<<values, 256, 0, stream>>>(
+        qlp, nullptr, nullptr, (const gd_bf16 *)w_uv, (const gd_bf16 *)gate, ldg, (gd_bf16 *)out, m, q);
     return (int)hipGetLastError();
 }

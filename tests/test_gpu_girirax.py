@@ -409,6 +409,18 @@ def test_latent_attention_of_prompts_portions_and_steps(backend, gda, arena, L, 
     _near(got, want, dtype, factor=1.5 if dtype == BF16 else 10)
 
 
+@pytest.mark.parametrize("tmax", [1024, 1025], ids=["8 pieces", "9 pieces"])
+@pytest.mark.parametrize("sizes", [(3, 72, 24, 56, 112), (17, 32, 16, 40, 64), (2, 136, 136, 96, 640)], ids=lambda s: "x".join(map(str, s)))
+def test_steps_whose_keys_are_cut_into_pieces(backend, gda, arena, L, sizes, tmax):
+    """Sequences that hold from one to all of their pieces, on both sides of the number of pieces that are merged with the value
+    up-projection, against the plain softmax over what the cache holds."""
+    la = Latent(gda, backend, arena, L, BF16, *sizes, tmax=tmax)
+    la.cache.write_float(la.rng.standard_normal(la.cache.shape))
+    for starts in ((0, tmax - 1, 128), (511, 127, 640), (1000, 0, 896)):
+        got, want = la.run([(slot, start, 1) for slot, start in enumerate(starts)])
+        _near(got, want, BF16, factor=1.5)
+
+
 @pytest.mark.parametrize("sizes", [(4, 72, 24, 56, 112), (16, 128, 64, 128, 512)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("form", ["expanded", "absorbed"])
 def test_every_key_is_seen_by_the_rows_behind_it_and_by_no_other(backend, gda, arena, L, sizes, form):
