@@ -9,8 +9,9 @@
  *            their latents (scores, weights and sums in F32)
  *   value    per token and head: the value up-projection of that sum, times the sigmoid of the output gate
  * They are the F32 path and the path of sizes outside the matrix-core kernels (latent_decode.hip, latent_prefill.hip).
- * Bound by round trips and by re-reading the up-projections for every row: elements are requested sixteen, outputs eight at a time,
- * with every sum in the order of the plain loop (390 rows, 8 heads, F32: query 47 -> 41, attend 132 -> 103, value 81 -> 67 us).
+ * Bound by round trips and by re-reading the up-projections: elements are requested sixteen, outputs four or eight at a time, and
+ * four rows share a reading where there are many, with every sum in the order of the plain loop (mean over portions of 160 to 570
+ * rows, 8 heads, F32: query 47 -> 24, attend 132 -> 103, value 81 -> 33 us).
  */
 #include "../../_shared/hip_device.h"
 #include "hip_latent_attention_types.h"
@@ -121,50 +122,64 @@ gd_latent_prepare_vec_kernel(const gd_bf16 *__restrict__ proj, uint32_t ld, cons
     for (uint32_t c = m.kv_rank + m.rot_dim + lane; c < m.pitch; c += 64u) dst[c] = (gd_bf16)0.f;
 }
 
-/* sum of q[i] * w[i] over n elements, ascending; a thread's own row in pieces of 16 bytes where it is aligned, sixteen elements
- * requested together */
-template <typename T>
-__device__ __forceinline__ float gd_latent_row_dot(const float *q, const T *__restrict__ w, uint32_t n)
+/* R sums of q[i] * w[i] over n elements, ascending, q's rows n floats apart; a thread's own row w in pieces of 16 bytes where it is
+ * aligned, sixteen elements requested together */
+template <int R, typename T>
+__device__ __forceinline__ void gd_latent_row_dot(const float *q, const T *__restrict__ w, uint32_t n, float (&a)[R])
 {
     constexpr uint32_t E = 16u / sizeof(T), PIECES = 16u / E;
     typedef T vec __attribute__((ext_vector_type(E)));
-    float a = 0.f;
     uint32_t i = 0u;
+#pragma unroll
+    for (int r = 0; r < R; ++r) a[r] = 0.f;
     if ((reinterpret_cast<uintptr_t>(w) & 15u) == 0u) {
         for (; i + 16u <= n; i += 16u) {
             vec v[PIECES];
 #pragma unroll
             for (uint32_t p = 0; p < PIECES; ++p) v[p] = *reinterpret_cast<const vec *>(w + i + p * E);
 #pragma unroll
-            for (uint32_t e = 0; e < 16u; ++e) a = fmaf(q[i + e], (float)v[e / E][e % E], a);
+            for (uint32_t e = 0; e < 16u; ++e)
+#pragma unroll
+                for (int r = 0; r < R; ++r) a[r] = fmaf(q[(uint32_t)r * n + i + e], (float)v[e / E][e % E], a[r]);
         }
     }
-    for (; i < n; ++i) a = fmaf(q[i], (float)w[i], a);
-    return a;
+    for (; i < n; ++i)
+#pragma unroll
+        for (int r = 0; r < R; ++r) a[r] = fmaf(q[(uint32_t)r * n + i], (float)w[i], a[r]);
 }
 
-/* grid (rows, heads); w_ukt [heads, kv_rank, dim]; ql [rows, heads, pitch] */
-template <typename T>
+/* grid (ceil(rows / R), heads); w_ukt [heads, kv_rank, dim]; ql [rows, heads, pitch].  R rows share a reading of the weights */
+template <typename T, int R>
 __global__ void __launch_bounds__(256)
 gd_latent_query_kernel(const T *__restrict__ qv, const T *__restrict__ w_ukt, const float *__restrict__ angles,
-                       T *__restrict__ ql, gd_hip_latent_params m)
+                       T *__restrict__ ql, gd_hip_latent_params m, uint32_t rows)
 {
-    extern __shared__ float sq[]; /* dim */
-    const uint32_t row = blockIdx.x, h = blockIdx.y, half = m.rot_dim / 2u;
-    const T *src = qv + ((size_t)row * m.heads + h) * (m.dim + m.rot_dim);
-    for (uint32_t d = threadIdx.x; d < m.dim; d += 256u) sq[d] = (float)src[d];
+    extern __shared__ float sq[]; /* [R][dim] */
+    const uint32_t row0 = blockIdx.x * R, h = blockIdx.y, half = m.rot_dim / 2u, n = min(rows - row0, (uint32_t)R);
+    for (uint32_t r = 0; r < R; ++r) { /* rows behind the last repeat it */
+        const T *src = qv + ((size_t)(row0 + min(r, n - 1u)) * m.heads + h) * (m.dim + m.rot_dim);
+        for (uint32_t d = threadIdx.x; d < m.dim; d += 256u) sq[r * m.dim + d] = (float)src[d];
+    }
     __syncthreads();
-    T *dst = ql + ((size_t)row * m.heads + h) * m.pitch;
     for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) {
-        dst[c] = (T)gd_latent_row_dot(sq, w_ukt + ((size_t)h * m.kv_rank + c) * m.dim, m.dim);
+        float a[R];
+        gd_latent_row_dot<R>(sq, w_ukt + ((size_t)h * m.kv_rank + c) * m.dim, m.dim, a);
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r)
+            if (r < n) ql[((size_t)(row0 + r) * m.heads + h) * m.pitch + c] = (T)a[r];
     }
-    for (uint32_t i = threadIdx.x; i < half; i += 256u) {
-        const float u = (float)src[m.dim + i], v = (float)src[m.dim + half + i];
-        const float c1 = angles[(size_t)row * m.rot_dim + i], s1 = angles[(size_t)row * m.rot_dim + half + i];
-        dst[m.kv_rank + i] = (T)(u * c1 - v * s1);
-        dst[m.kv_rank + half + i] = (T)(v * c1 + u * s1);
+    for (uint32_t r = 0; r < n; ++r) {
+        const uint32_t row = row0 + r;
+        const T *src = qv + ((size_t)row * m.heads + h) * (m.dim + m.rot_dim);
+        T *dst = ql + ((size_t)row * m.heads + h) * m.pitch;
+        for (uint32_t i = threadIdx.x; i < half; i += 256u) {
+            const float u = (float)src[m.dim + i], v = (float)src[m.dim + half + i];
+            const float c1 = angles[(size_t)row * m.rot_dim + i], s1 = angles[(size_t)row * m.rot_dim + half + i];
+            dst[m.kv_rank + i] = (T)(u * c1 - v * s1);
+            dst[m.kv_rank + half + i] = (T)(v * c1 + u * s1);
+        }
+        for (uint32_t c = m.kv_rank + m.rot_dim + threadIdx.x; c < m.pitch; c += 256u) dst[c] = (T)0.f;
     }
-    for (uint32_t c = m.kv_rank + m.rot_dim + threadIdx.x; c < m.pitch; c += 256u) dst[c] = (T)0.f;
 }
 
 /* grid (rows, heads); o_lat F32 [rows, heads, kv_rank] */
@@ -188,7 +203,11 @@ gd_latent_attend_kernel(const T *__restrict__ ql, const T *__restrict__ cache, f
         __syncthreads();
         const uint32_t k = k0 + threadIdx.x;
         float score = -INFINITY;
-        if (k < keys) score = gd_latent_row_dot(sq, rows + (size_t)k * m.pitch, used) * m.scale;
+        if (k < keys) {
+            float a[1];
+            gd_latent_row_dot<1>(sq, rows + (size_t)k * m.pitch, used, a);
+            score = a[0] * m.scale;
+        }
         /* maximum of the block's scores */
         float t = gd_wave_max(score);
         if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = t;
@@ -220,41 +239,62 @@ gd_latent_attend_kernel(const T *__restrict__ ql, const T *__restrict__ cache, f
         o_lat[((size_t)row * m.heads + h) * m.kv_rank + c] = so[c] / total;
 }
 
-/* grid (rows, heads); out [rows, heads * vdim] */
-template <typename T>
+/* grid (ceil(rows / R), heads); out [rows, heads * vdim].  R rows share a reading of the weights; a wavefront takes every fourth
+ * output, OUTS of them at a time: their loads and their exchanges overlap */
+template <typename T, int R>
 __global__ void __launch_bounds__(256)
 gd_latent_value_kernel(const float *__restrict__ o_lat, const T *__restrict__ w_uv, const T *__restrict__ gate,
-                       uint32_t ldg, T *__restrict__ out, gd_hip_latent_params m)
+                       uint32_t ldg, T *__restrict__ out, gd_hip_latent_params m, uint32_t rows)
 {
-    extern __shared__ float so[]; /* kv_rank */
-    constexpr uint32_t OUTS = 8u;
-    const uint32_t row = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
-    for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) so[c] = o_lat[((size_t)row * m.heads + h) * m.kv_rank + c];
+    extern __shared__ float so[]; /* [R][kv_rank] */
+    constexpr uint32_t OUTS = R == 1 ? 8u : 4u;
+    const uint32_t row0 = blockIdx.x * R, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    const uint32_t n = min(rows - row0, (uint32_t)R);
+    for (uint32_t r = 0; r < R; ++r) { /* rows behind the last repeat it */
+        const float *src = o_lat + ((size_t)(row0 + min(r, n - 1u)) * m.heads + h) * m.kv_rank;
+        for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) so[r * m.kv_rank + c] = src[c];
+    }
     __syncthreads();
-    /* a wavefront takes every fourth output, eight of them at a time: their loads and their exchanges overlap */
     for (uint32_t v0 = wave; v0 < m.vdim; v0 += 4u * OUTS) {
         const T *w = w_uv + ((size_t)h * m.vdim + v0) * m.kv_rank;
-        float a[OUTS], g[OUTS];
+        float a[OUTS][R];
 #pragma unroll
-        for (uint32_t i = 0; i < OUTS; ++i) {
-            a[i] = 0.f;
-            g[i] = (float)gate[(size_t)row * ldg + h * m.vdim + min(v0 + 4u * i, m.vdim - 1u)];
-        }
+        for (uint32_t i = 0; i < OUTS; ++i)
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[i][r] = 0.f;
         for (uint32_t c = lane; c < m.kv_rank; c += 64u) {
+            float x[OUTS];
 #pragma unroll
-            for (uint32_t i = 0; i < OUTS; ++i)
-                a[i] = fmaf(so[c], (float)w[(size_t)min(4u * i, m.vdim - 1u - v0) * m.kv_rank + c], a[i]);
+            for (uint32_t i = 0; i < OUTS; ++i) x[i] = (float)w[(size_t)min(4u * i, m.vdim - 1u - v0) * m.kv_rank + c];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const float o = so[(uint32_t)r * m.kv_rank + c];
+#pragma unroll
+                for (uint32_t i = 0; i < OUTS; ++i) a[i][r] = fmaf(o, x[i], a[i][r]);
+            }
         }
 #pragma unroll
-        for (uint32_t i = 0; i < OUTS; ++i) a[i] = gd_wave_sum(a[i]);
+        for (uint32_t i = 0; i < OUTS; ++i)
 #pragma unroll
-        for (uint32_t i = 0; i < OUTS; ++i) {
-            const uint32_t v = v0 + 4u * i;
-            if (lane == 0u && v < m.vdim)
-                out[(size_t)row * m.heads * m.vdim + h * m.vdim + v] = (T)(a[i] * gd_sigmoid_f32(g[i]));
+            for (int r = 0; r < R; ++r) a[i][r] = gd_wave_sum(a[i][r]);
+        /* lane r * OUTS + i stores output i of row r */
+        float mine = 0.f;
+#pragma unroll
+        for (uint32_t i = 0; i < OUTS; ++i)
+#pragma unroll
+            for (uint32_t r = 0; r < R; ++r)
+                if (lane == r * OUTS + i) mine = a[i][r];
+        const uint32_t r = lane / OUTS, v = v0 + 4u * (lane % OUTS);
+        if (r < n && v < m.vdim) {
+            const float g = (float)gate[(size_t)(row0 + r) * ldg + h * m.vdim + v];
+            out[(size_t)(row0 + r) * m.heads * m.vdim + h * m.vdim + v] = (T)(mine * gd_sigmoid_f32(g));
         }
     }
 }
+
+/* four rows to a workgroup where that leaves two workgroups for every compute unit of the chip (six portions of 160 to 570 rows, 8 heads,
+ * three of them shared, mean: value 67 -> 33, query 41 -> 24 us), one otherwise, so that every unit has work */
+static bool gd_latent_rows_share(uint32_t rows, uint32_t heads) { return (uint64_t)rows * heads >= 4u * 512u; }
 
 extern "C" int gd_hip_launch_latent_prepare(hipStream_t stream, const void *proj, uint32_t ld, const float *q_norm,
                                             const float *kv_norm, const float *freq, float *angles, void *cq, void *cache,
@@ -276,9 +316,9 @@ extern "C" int gd_hip_launch_latent_prepare(hipStream_t stream, const void *proj
 extern "C" int gd_hip_launch_latent_query(hipStream_t stream, const void *qv, const void *w_ukt, const float *angles,
                                           void *ql, const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32)
 {
-    const dim3 grid(q->rows, m->heads);
-#define GD_GO(T) gd_latent_query_kernel<T><<<grid, 256, m->dim * sizeof(float), stream>>>((const T *)qv, (const T *)w_ukt, angles, (T *)ql, *m)
-    if (is_f32) GD_GO(float); else GD_GO(gd_bf16);
+#define GD_GO(T, R) gd_latent_query_kernel<T, R><<<dim3((q->rows + R - 1u) / R, m->heads), 256, R * m->dim * sizeof(float), stream>>>((const T *)qv, (const T *)w_ukt, angles, (T *)ql, *m, q->rows)
+    if (gd_latent_rows_share(q->rows, m->heads) && m->dim <= 2048u) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
+    else { if (is_f32) GD_GO(float, 1); else GD_GO(gd_bf16, 1); }
 #undef GD_GO
     return (int)hipGetLastError();
 }
@@ -299,10 +339,10 @@ extern "C" int gd_hip_launch_latent_attend(hipStream_t stream, const void *ql, c
 extern "C" int gd_hip_launch_latent_value(hipStream_t stream, const float *o_lat, const void *w_uv, const void *gate,
                                           uint32_t ldg, void *out, uint32_t rows, const gd_hip_latent_params *m, int is_f32)
 {
-    const dim3 grid(rows, m->heads);
     if (rows == 0u) return (int)hipSuccess;
-#define GD_GO(T) gd_latent_value_kernel<T><<<grid, 256, m->kv_rank * sizeof(float), stream>>>(o_lat, (const T *)w_uv, (const T *)gate, ldg, (T *)out, *m)
-    if (is_f32) GD_GO(float); else GD_GO(gd_bf16);
+#define GD_GO(T, R) gd_latent_value_kernel<T, R><<<dim3((rows + R - 1u) / R, m->heads), 256, R * m->kv_rank * sizeof(float), stream>>>(o_lat, (const T *)w_uv, (const T *)gate, ldg, (T *)out, *m, rows)
+    if (gd_latent_rows_share(rows, m->heads)) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
+    else { if (is_f32) GD_GO(float, 1); else GD_GO(gd_bf16, 1); }
 #undef GD_GO
     return (int)hipGetLastError();
 }
