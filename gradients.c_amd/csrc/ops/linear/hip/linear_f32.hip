@@ -86,9 +86,11 @@ gd_linear_f32_kernel(const float *__restrict__ x, const float *__restrict__ w, c
  *   SPLIT true   all four on one 32 x 32 tile, a quarter of K each, stages of their own and no barrier, summed in wavefront
  *                order at the end: four times as many tiles for outputs that would leave compute units without one, and the
  *                form of few rows, where the weights' bytes decide
+ * Both add the same quarters of K in the same order (the first form closes its sums where a quarter ends), so that a row has
+ * the same bits whatever rows are beside it: a token replayed alone is the token of the portion.
  * Measured against gd_linear_f32_kernel (us): 6 x 1024 -> 32768 25.9 (151; 5.2 TB/s of weights),
- * 6 x 2816 -> 1024 15.9 (308), 390 x 1024 -> 4384 42 (184; 83 TFLOP/s), 390 x 2816 -> 1024 29 (412), 390 x 1024 -> 2816 gated 71
- * (217), 4096 x 1024 -> 4384 326 (730; 113 TFLOP/s).  Error against 64 bits of a decoder's logits 8e-7 (1.2e-6).
+ * 6 x 2816 -> 1024 15.9 (308), 390 x 1024 -> 4384 42 (184; 83 TFLOP/s), 390 x 2816 -> 1024 29 (412), 390 x 1024 -> 2816 gated 74
+ * (217; 72 with one running sum), 4096 x 1024 -> 4384 337 (730; 331 with one running sum; 109 TFLOP/s).  Error against 64 bits of a decoder's logits 8e-7 (1.2e-6).
  */
 typedef float gd_f32x16 __attribute__((ext_vector_type(16)));
 
@@ -141,11 +143,11 @@ gd_linear_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__
     const uint32_t fr = lane & 31u, fh = lane >> 5;
     const uint32_t a_row = (SPLIT ? 0u : (wave >> 1) * 32u) + fr, b_row = TILE + (SPLIT ? 0u : (wave & 1u) * 32u) + fr;
     const uint32_t swizzle = (fr & 7u) ^ ((fr >> 3) & 1u);
-    gd_f32x16 acc[GATED ? 2 : 1];
+    gd_f32x16 acc[GATED ? 2 : 1], sums[GATED ? 2 : 1]; /* of a quarter of K; !SPLIT: of the quarters so far */
 #pragma unroll
     for (int g = 0; g < (GATED ? 2 : 1); ++g)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[g][e] = 0.f;
+        for (int e = 0; e < 16; ++e) acc[g][e] = sums[g][e] = 0.f;
     auto multiply = [&](uint32_t stage) __attribute__((always_inline)) {
         const gd_float4 *s = reinterpret_cast<const gd_float4 *>(s_mem + own + stage * (ROWS * 128u));
         gd_float4 a[4], b[GATED ? 2 : 1][4];
@@ -182,18 +184,28 @@ gd_linear_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__
         request(0u, 0u);
         if (1u < blocks) request(1u, 1u);
         uint32_t stage = 0u, next = 2u;
-        for (uint32_t kb = 0; kb < blocks; ++kb) {
-            /* this wavefront's loads of block kb have landed once only those of block kb + 1 are outstanding; behind the barrier
-             * everybody's have, and everybody has read block kb - 1, whose stage is filled next */
-            if (kb + 1u >= blocks) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            else if (GATED) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if (kb + 2u < blocks) request(kb + 2u, next);
-            multiply(stage);
-            stage = stage + 1u == STAGES ? 0u : stage + 1u;
-            next = next + 1u == STAGES ? 0u : next + 1u;
+#pragma unroll 1
+        for (uint32_t quarter = 0, kb = 0; quarter < 4u; ++quarter) {
+            for (const uint32_t end = blocks * (quarter + 1u) / 4u; kb < end; ++kb) {
+                /* this wavefront's loads of block kb have landed once only those of block kb + 1 are outstanding; behind the
+                 * barrier everybody's have, and everybody has read block kb - 1, whose stage is filled next */
+                if (kb + 1u >= blocks) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                else if (GATED) asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)" ::: "memory");
+                else asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                if (kb + 2u < blocks) request(kb + 2u, next);
+                multiply(stage);
+                stage = stage + 1u == STAGES ? 0u : stage + 1u;
+                next = next + 1u == STAGES ? 0u : next + 1u;
+            }
+#pragma unroll
+            for (int g = 0; g < (GATED ? 2 : 1); ++g)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    sums[g][e] += acc[g][e];
+                    acc[g][e] = 0.f;
+                }
         }
     }
     static_assert(ITEMS == (SPLIT ? (GATED ? 12 : 8) : (GATED ? 6 : 4)), "the waits above count the loads of a stage");
@@ -205,7 +217,7 @@ gd_linear_f32_mfma_kernel(const float *__restrict__ x, const float *__restrict__
 #pragma unroll
             for (uint32_t r = 0; r < 16u; ++r) {
                 const uint32_t m = row0 + 8u * (r / 4u) + r % 4u;
-                if (m < p.M) y[(size_t)m * p.ldy + n] = gd_f32_output<GATED>(acc[0][r], acc[GATED ? 1 : 0][r], bias, n, p);
+                if (m < p.M) y[(size_t)m * p.ldy + n] = gd_f32_output<GATED>(sums[0][r], sums[GATED ? 1 : 0][r], bias, n, p);
             }
         }
         return;

@@ -71,6 +71,29 @@ def test_32_bit_projections_on_the_matrix_cores(backend, gda, arena, M, N, K):
     _near(half.read(), want[:, :N] * gate / (1 + np.exp(-gate)), F32)
 
 
+@pytest.mark.parametrize("M,N,K", [(1030, 2000, 352), (1025, 1090, 32), (1100, 1100, 96)])
+def test_a_32_bit_row_does_not_depend_on_the_rows_beside_it(backend, gda, arena, M, N, K):
+    """Rows of a call that fills the chip with 64 x 64 tiles (whose stages are used again and again) against the same rows in
+    calls of few: the same sums in the same order, plain and gated."""
+    rng = np.random.default_rng(N)
+    x, xv = _put(arena, F32, rng.standard_normal((M, K)))
+    w, wv = _put(arena, F32, rng.standard_normal((2 * N, K)) / np.sqrt(K))
+    b, bv = _put(arena, F32, rng.standard_normal(2 * N))
+    y, half = arena.alloc((M, 2 * N), F32), arena.alloc((M, N), F32)
+    backend.fused_linear(x, w, b, None, None, y, True, 1, 0)
+    backend.fused_linear(x, w, b, None, None, half, True, 1, 0, epilogue=1)
+    all_rows, gated = y.read(), half.read()
+    want = xv @ wv.T + bv
+    _near(all_rows, want, F32)
+    _near(gated, want[:, :N] * want[:, N:] / (1 + np.exp(-want[:, N:])), F32)
+    for first, n in ((0, 1), (M - 33, 33), (61, 40)):
+        few, part = arena.alloc((n, 2 * N), F32), arena.alloc((n, N), F32)
+        backend.fused_linear(x.rows(first, n), w, b, None, None, few, True, 1, 0)
+        backend.fused_linear(x.rows(first, n), w, b, None, None, part, True, 1, 0, epilogue=1)
+        assert np.array_equal(few.read(), all_rows[first:first + n])
+        assert np.array_equal(part.read(), gated[first:first + n])
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 8200, 512), (16, 4099, 1024), (17, 4099, 1024), (33, 3073, 1024), (65, 12301, 512), (40, 2050, 2048),
                                    (3, 3100, 4096), (64, 1600, 4096)])
 def test_few_rows_onto_many_columns(backend, gda, arena, M, N, K):
