@@ -6,7 +6,7 @@
  * One workgroup owns a [N, COLS] column slice of one head of one sequence and keeps it in registers: thread (r, l) holds
  * rows r, r + R, ... (R = 1024 / COLS) of columns 4l .. 4l+3, so a state row is read and written in whole 128-byte lines.  Tokens come
  * in batches through LDS; the column sums of S^T C go through wavefront shuffles and one LDS exchange
- * per batch.  This is the decode step (HBM-bound on reading and writing S once), the whole F32 path and the path of
+ * per batch, in the same order for 32 and 64 columns, so that a token has the same bits in a step and in a portion.  This is the decode step (HBM-bound on reading and writing S once), the whole F32 path and the path of
  * short portions; long BF16 prompts take the matrix-core kernel of ssm_scan_chunk.hip.
  *
  * A sequence that starts at position 0 starts from a zero state, whatever its slot holds.
@@ -55,8 +55,9 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
 {
     constexpr uint32_t GD_SSM_BATCH = CONV ? 1u : 8u, GD_SSM_COLS = COLS;
     constexpr uint32_t L = GD_SSM_COLS / 4u, R = 256u / L, NS = NR * R; /* lanes of a row, rows of a pass, rows of all */
+    constexpr uint32_t HALVES = GD_SSM_COLS / 32u; /* passes that make 32 rows: a sum for each, the rows a multiple of 32 apart */
     __shared__ __align__(16) float sb[GD_SSM_BATCH][NS], sc[GD_SSM_BATCH][NS], sx[GD_SSM_BATCH][GD_SSM_COLS];
-    __shared__ __align__(16) float part[GD_SSM_BATCH][4][GD_SSM_COLS], sdt[GD_SSM_BATCH], sdec[GD_SSM_BATCH];
+    __shared__ __align__(16) float part[GD_SSM_BATCH][HALVES * 4u][GD_SSM_COLS], sdt[GD_SSM_BATCH], sdec[GD_SSM_BATCH];
     const uint32_t p0 = blockIdx.x * GD_SSM_COLS, h = blockIdx.y;
     const uint32_t l = threadIdx.x % L, r = threadIdx.x / L, wave = threadIdx.x >> 6;
     const uint32_t N = m.state, P = m.vdim, inner = m.heads * P, g = h / (m.heads / m.groups);
@@ -114,30 +115,39 @@ gd_ssm_scan_kernel(const T *__restrict__ xbc, const T *__restrict__ dt_raw, cons
         for (uint32_t t = 0; t < nb; ++t) {
             const float dec = sdec[t], dt = sdt[t];
             const gd_float4 x4 = *reinterpret_cast<const gd_float4 *>(&sx[t][4u * l]);
-            gd_float4 acc = {0.f, 0.f, 0.f, 0.f};
+            gd_float4 acc[HALVES] = {};
 #pragma unroll
             for (int i = 0; i < NR; ++i) {
                 const float b = dt * sb[t][r + R * i], c = sc[t][r + R * i];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     S[i][e] = fmaf(dec, S[i][e], b * x4[e]);
-                    acc[e] = fmaf(S[i][e], c, acc[e]);
+                    acc[i % (int)HALVES][e] = fmaf(S[i][e], c, acc[i % (int)HALVES][e]);
                 }
             }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (L <= 8u) acc[e] += __shfl_xor(acc[e], 8, 64);
-                acc[e] += __shfl_xor(acc[e], 16, 64);
-                acc[e] += __shfl_xor(acc[e], 32, 64);
+            for (uint32_t u = 0; u < HALVES; ++u) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (L <= 8u) acc[u][e] += __shfl_xor(acc[u][e], 8, 64);
+                    acc[u][e] += __shfl_xor(acc[u][e], 16, 64);
+                    acc[u][e] += __shfl_xor(acc[u][e], 32, 64);
+                }
+                if ((threadIdx.x & 63u) < L) *reinterpret_cast<gd_float4 *>(&part[t][u * 4u + wave][4u * l]) = acc[u];
             }
-            if ((threadIdx.x & 63u) < L) *reinterpret_cast<gd_float4 *>(&part[t][wave][4u * l]) = acc;
         }
         __syncthreads();
         for (uint32_t i = threadIdx.x; i < nb * GD_SSM_COLS; i += 256u) {
             const uint32_t t = i / GD_SSM_COLS, c = i % GD_SSM_COLS;
+            float eight[4]; /* of rows 0-7, 8-15, 16-23 and 24-31 of every 32: HALVES wavefronts each */
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                eight[k] = part[t][k * HALVES][c];
+                if (HALVES == 2u) eight[k] += part[t][k * HALVES + HALVES - 1u][c];
+            }
             if (c < cols)
                 y[(size_t)(first + t0 + (int32_t)t) * inner + h * P + p0 + c] =
-                    (T)(part[t][0][c] + part[t][1][c] + part[t][2][c] + part[t][3][c] + skip * sx[t][c]);
+                    (T)(eight[0] + eight[1] + eight[2] + eight[3] + skip * sx[t][c]);
         }
         __syncthreads();
     }
@@ -157,9 +167,12 @@ extern "C" int gd_hip_launch_ssm_scan(hipStream_t stream, const void *xbc, const
                                       const gd_hip_ssm_params *m, const gd_hip_ssm_conv *cv, const gd_hip_seqs *q,
                                       int is_f32)
 {
-    /* a decode step over whole 64-column slices: half as many workgroups convolve the B and C of their group once more, and each has
-     * twice the state on its way (64 sequences x 32 heads of [128, 64]: 38.4 -> 32.1 us, 4.2 TB/s of state) */
-    const bool pair = cv != nullptr && (m->vdim % 64u) == 0u && m->state <= 256u;
+    /* A decode step over whole 64-column slices: half as many workgroups convolve the B and C of their group once more, and each has
+     * twice the state on its way ([128, 64] states, us against 32 columns: 64 sequences x 32 heads 34.4 (40.0), x 128 heads 133
+     * (147), one sequence of 32 heads 6.2 (6.4); [64, 128] x 32 heads 36.1 (43.3) and 4.9 (4.9)).  Not for longer columns, whose 64
+     * state registers a lane leave too few wavefronts ([256, 64] x 64 heads: 1 sequence 11.8 (7.3), 8 sequences 23.1 (20.1), 64
+     * sequences 173 (144)) */
+    const bool pair = cv != nullptr && (m->vdim % 64u) == 0u && m->state <= 128u;
     const uint32_t slice = pair ? 64u : 32u;
     const dim3 grid((m->vdim + slice - 1u) / slice, m->heads, q->seqs);
     if (q->rows == 0u || q->seqs == 0u) return (int)hipSuccess;
@@ -178,8 +191,7 @@ extern "C" int gd_hip_launch_ssm_scan(hipStream_t stream, const void *xbc, const
     do {                                                                                                                            \
         const T *xt = (const T *)xbc, *dt = (const T *)dt_raw;                                                                      \
         if (m->state <= 64u) gd_ssm_scan_kernel<T, 4, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q);       \
-        else if (m->state <= 128u) gd_ssm_scan_kernel<T, 8, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q); \
-        else gd_ssm_scan_kernel<T, 16, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q);                      \
+        else gd_ssm_scan_kernel<T, 8, true, 64><<<grid, 256, 0, stream>>>(xt, dt, dt_bias, a_log, d_skip, states, (T *)y, *m, *cv, *q);                       \
     } while (0)
     if (pair) {
         if (is_f32) GD_PAIR(float); else GD_PAIR(gd_bf16);

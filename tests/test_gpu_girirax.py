@@ -330,6 +330,32 @@ def test_fused_step_over_64_column_slices(backend, gda, arena, dtype, H, P, N, G
     test_fused_convolution_and_recurrence_step(backend, gda, arena, dtype, H, P, N, Gn, K)
 
 
+@pytest.mark.parametrize("B", [1, 3, 70], ids=lambda b: "%d sequences" % b)
+@pytest.mark.parametrize("H,P,N", [(2, 64, 33), (3, 20, 40), (3, 128, 128), (4, 64, 256), (1, 192, 64)])
+def test_a_32_bit_token_has_the_same_bits_in_a_step_and_in_a_portion(backend, gda, arena, H, P, N, B):
+    """The fused launch and the two operators, which take portions, add in the same order, however many sequences there are."""
+    rng = np.random.default_rng(H * P + N)
+    ch, K = H * P + 2 * N, 4
+    rest = [_put(arena, F32, v)[0].view() for v in (rng.uniform(-3, -1, H), rng.uniform(-1, 1, H), rng.standard_normal(H))]
+    taps, bias = _put(arena, F32, rng.standard_normal((ch, K)) * 0.5)[0], _put(arena, F32, rng.standard_normal(ch) * 0.1)[0]
+    args = gda.SsmArgs(H, P, N, 1)
+    used = rng.standard_normal((B, K, ch)), rng.standard_normal((B, H, N, P))
+    x = _put(arena, F32, rng.standard_normal((B, ch + H)))[0]
+    xm, dt = x.matrix(cols=ch), x.matrix(cols=H)
+    dt.offset += ch * x.itemsize
+    sq = Seqs(gda, arena, [(b, 9, 1) for b in range(B)])
+    sides = [(_put(arena, F32, used[0])[0], _put(arena, F32, used[1])[0], arena.alloc((B, H * P), F32)) for _ in range(2)]
+    conv = arena.alloc((B, ch), F32)
+    ring, st, y = sides[0]
+    _ok(backend.call("gd_backend_causal_conv_silu", xm, taps.view(), bias.view(), ring.view(), conv.view(), sq.ref()))
+    _ok(backend.call("gd_backend_ssm_scan", conv.view(), dt, *rest, st.view(), y.view(), sq.ref(), C.byref(args)))
+    ring, st, y = sides[1]
+    _ok(backend.call("gd_backend_conv_ssm_step", xm, taps.view(), bias.view(), ring.view(), dt, *rest, st.view(), y.view(),
+                     sq.ref(), C.byref(args)))
+    for a, b in zip(*sides):
+        assert np.array_equal(a.read(), b.read())
+
+
 @TYPES
 @pytest.mark.parametrize("inner,parts", [(64, 1), (96, 4), (4096, 2), (30, 3), (5000, 1)])
 def test_gate_then_group_norm(backend, gda, arena, L, dtype, inner, parts):
