@@ -5,7 +5,7 @@
  *   absorb  q_lat[h] = W_uk[h]^T q[h] per 16 rows, head and 64 latent columns, and the rotated query part behind it
  *   attend  a workgroup of 4 wavefronts takes 16 or 32 heads of one token over a piece of its keys: a cache row is read from
  *           memory once for all of them.  HBM-bound on the cache rows.
- *   merge   the pieces of a token and head into one latent vector (where there are few, a part of value)
+ *   merge   the pieces of a token and head into one latent vector (a part of value where that reads little again)
  *   value   16 tokens and one head: the value up-projection and the output gate
  *
  * attend.  Keys advance in tiles of 32 rows through two LDS stages filled by global -> LDS loads; two workgroups share a
@@ -31,10 +31,21 @@
 
 #define GD_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0)
 #define GD_LD_TILE 32u
-/* pieces up to which the value kernel merges them itself: one launch less, while each of its ceil(vdim / 32) workgroups per head
- * reads the pieces again (64 rows, 8 heads, vdim 128, kv_rank 256: 7.3 us against 5.0 + 4.8); more pieces come with few rows,
- * where the merge kernel spreads their latents over more wavefronts */
-#define GD_LD_FOLD 8u
+/* Pieces that the value kernel can merge itself: one launch less, while each of its ceil(vdim / 32) workgroups per head reads the
+ * pieces again, one round trip after the other.  Taken where that is little per workgroup and in all; the whole call against a
+ * merge launch (dim and vdim 128; us):
+ *   kv_rank 256, 8 heads   1 row: 1 piece 13.0 (14.5), 4 pieces 14.2 (15.1), 8 pieces 15.9 (14.9)
+ *                          16 rows: 2 pieces 15.5 (16.2), 3 pieces 17.6 (17.8), 8 pieces 23.3 (18.3)
+ *                          64 rows: 2 pieces 17.6 (18.4), 3 pieces 19.9 (19.1), 8 pieces 28.2 (23.8)
+ *   kv_rank 256, 32 heads  64 rows: 1 piece 23.7 (24.7), 2 pieces 27.6 (26.6)
+ *   kv_rank 512, 16 heads  1 row: 2 pieces 17.0 (18.2), 3 pieces 18.7 (18.6);  64 rows: 1 piece 23.8 (24.5), 2 pieces 26.6 (26.2) */
+#define GD_LD_FOLD 4u
+static bool gd_latent_folds(const gd_hip_latent_params &m, uint32_t rows)
+{
+    const uint32_t reads = m.pieces * m.kv_rank; /* F32 values per workgroup and row */
+    if (m.pieces > GD_LD_FOLD) return false;
+    return rows <= 4u ? reads <= 1024u : reads <= 512u && (m.pieces == 1u || (uint64_t)rows * m.heads <= 1024u);
+}
 
 /* grid (ceil(kv_rank / 64) + 1, heads, ceil(rows / 16)); dim % 8 == 0, rot_dim % 8 == 0 (16-byte fragments of q).  A chain of round
  * trips, so the fragments of four steps are requested together and the rotated part has a workgroup of its own, the last of x
@@ -341,31 +352,23 @@ gd_latent_value_mfma_kernel(const gd_bf16 *__restrict__ merged, const float *__r
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         g[r] = (float)gate[(size_t)min(r0 + 4u * lg + (uint32_t)r, rows - 1u) * ldg + h * m.vdim + min(v0 + li, m.vdim - 1u)];
-    /* PIECES: lane group lg holds the weights of pieces lg and 4 + lg of its lane's row */
+    /* PIECES: lane group lg holds the weight of piece lg of its lane's row */
     uint32_t live = 0u;
-    float weight[2] = {0.f, 0.f};
+    float weight = 0.f;
     if (PIECES) {
         int32_t seq, pos, slot;
         if (gd_seq_of_row(q, own, &seq, &pos, &slot))
             live = min((min((uint32_t)pos + 1u, m.tmax) + m.piece_keys - 1u) / m.piece_keys, m.pieces);
-        float ref[2], part[2];
-#pragma unroll
-        for (uint32_t i = 0; i < 2u; ++i) {
-            const bool has = 4u * i + lg < live;
-            const float *v = ml + (((size_t)own * m.pieces + (has ? 4u * i + lg : 0u)) * m.heads + h) * 2u;
-            ref[i] = has ? v[0] : -INFINITY;
-            part[i] = has ? v[1] : 0.f;
-        }
-        float top = fmaxf(ref[0], ref[1]);
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const bool has = lg < live;
+        const float *v = ml + (((size_t)own * m.pieces + (has ? lg : 0u)) * m.heads + h) * 2u;
+        const float ref = has ? v[0] : -INFINITY, part = has ? v[1] : 0.f;
+        float top = fmaxf(ref, __shfl_xor(ref, 32, 64));
         top = fmaxf(top, __shfl_xor(top, 16, 64));
-#pragma unroll
-        for (uint32_t i = 0; i < 2u; ++i) weight[i] = 4u * i + lg < live ? __builtin_amdgcn_exp2f(ref[i] - top) : 0.f;
-        float total = weight[0] * part[0] + weight[1] * part[1];
+        weight = has ? __builtin_amdgcn_exp2f(ref - top) : 0.f;
+        float total = weight * part;
         total += __shfl_xor(total, 32, 64);
         total += __shfl_xor(total, 16, 64);
-        weight[0] /= total;
-        weight[1] /= total;
+        weight /= total;
     }
     gd_float4 acc = {0.f, 0.f, 0.f, 0.f};
     for (uint32_t s = s_begin; s < s_end; s += 4u) { /* the loads of four steps together */
@@ -397,9 +400,8 @@ gd_latent_value_mfma_kernel(const gd_bf16 *__restrict__ merged, const float *__r
                     }
 #pragma unroll
                 for (uint32_t i = 0; i < 2u; ++i) {
-                    const uint32_t from = li + 16u * ((p + i) & 3u);
-                    const float w0 = __shfl(weight[0], (int)from, 64), w1 = __shfl(weight[1], (int)from, 64);
-                    const float w = p + i < live ? (p + i < 4u ? w0 : w1) : 0.f;
+                    const float of_piece = __shfl(weight, (int)(li + 16u * ((p + i) & 3u)), 64);
+                    const float w = p + i < live ? of_piece : 0.f;
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -466,7 +468,7 @@ extern "C" int gd_hip_launch_latent_decode(hipStream_t stream, const void *qv, c
 #undef GD_GO
     if (e != 0) return e;
     const dim3 values((m.vdim + 31u) / 32u, m.heads, rt);
-    if (m.pieces <= GD_LD_FOLD) {
+    if (gd_latent_folds(m, q.rows)) {
         gd_latent_value_mfma_kernel<true><<<values, 256, 0, stream>>>(
             nullptr, o_part, ml, (const gd_bf16 *)w_uv, (const gd_bf16 *)gate, ldg, (gd_bf16 *)out, m, q);
         return (int)hipGetLastError();

@@ -470,6 +470,18 @@ def test_steps_whose_keys_are_cut_into_pieces(backend, gda, arena, L, sizes, tma
         _near(got, want, BF16, factor=1.5)
 
 
+@pytest.mark.parametrize("rows,tmax,sizes", [(3, 500, (3, 72, 24, 56, 112)), (3, 520, (3, 72, 24, 56, 112)), (4, 256, (2, 40, 16, 32, 512)),
+                                             (5, 256, (2, 40, 16, 32, 512)), (4, 500, (5, 32, 16, 40, 256)), (64, 256, (16, 16, 8, 32, 64)),
+                                             (65, 256, (16, 16, 8, 32, 64)), (70, 128, (20, 16, 8, 48, 128)), (17, 200, (4, 24, 8, 40, 240))],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_steps_on_both_sides_of_the_merge_with_the_value(backend, gda, arena, L, rows, tmax, sizes):
+    """One to five pieces, few rows and many, sequences of every length down to one key: merged by a launch of their own or not."""
+    la = Latent(gda, backend, arena, L, BF16, *sizes, slots=rows, tmax=tmax)
+    la.cache.write_float(la.rng.standard_normal(la.cache.shape))
+    got, want = la.run([(slot, (tmax - 1) * (rows - 1 - slot) // (rows - 1), 1) for slot in range(rows)])
+    _near(got, want, BF16, factor=1.5)
+
+
 @pytest.mark.parametrize("sizes", [(4, 72, 24, 56, 112), (16, 128, 64, 128, 512)], ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("form", ["expanded", "absorbed"])
 def test_every_key_is_seen_by_the_rows_behind_it_and_by_no_other(backend, gda, arena, L, sizes, form):
