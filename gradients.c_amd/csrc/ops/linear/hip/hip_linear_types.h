@@ -17,6 +17,7 @@
 #define GD_HIP_LINEAR_Y_F32 2u     /* y is F32 (BF16 operands) */
 #define GD_HIP_LINEAR_CLAMPED_GATE 4u /* swiglu_cols: g sigmoid(gate_alpha g) (v + 1), both kept within gate_limit */
 #define GD_HIP_LINEAR_SQUARE_RELU 8u  /* not gated: y = max(u, 0)^2 */
+#define GD_HIP_LINEAR_STREAM_Y 16u    /* tile kernel: y is stored past the L2s (set by its launcher) */
 
 typedef struct gd_hip_linear_params {
     uint32_t M, N, K;
@@ -44,7 +45,7 @@ typedef struct gd_hip_linear_params {
      * tile count on a second line every projection launch of a decode step took 0.06 us longer. */
     uint16_t force_tiles, force_waves; /* tunables: 0 = automatic */
     uint16_t no_lds_stream;            /* tunable: 1 = weights always go straight to registers */
-    uint16_t flags;                    /* GD_HIP_LINEAR_* below; the BF16 and F32 kernels only, 0 for F16 operands */
+    uint16_t flags;                    /* GD_HIP_LINEAR_* above; 0 for F16 operands (but for GD_HIP_LINEAR_STREAM_Y) */
 } gd_hip_linear_params;
 #ifdef __cplusplus
 static_assert(sizeof(gd_hip_linear_params) == 76, "the few-row kernel's arguments must stay within one 128-byte line");

@@ -678,10 +678,21 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         c.u[3] = s1[1];
         return c.h;
     };
-    /* Streaming stores: all compute units end their tiles together, and 128 KB from each of them would wait for the write-back of
-     * as many dirty lines of the L2s (a launch without any store is a tenth shorter).  BF16, us: 30229 x 2048 -> 11264 1174 ->
-     * 1133, 27000 x 4096 -> 16896 3106 -> 2967, 16000 x 512 -> 1536 40.9 -> 38.6 */
-    auto store_own = [&](gd_elem8 h, gd_elem *at) __attribute__((always_inline)) { __builtin_nontemporal_store(h, reinterpret_cast<gd_elem8 *>(at)); };
+    /* Streaming stores where the launcher asks for them: all compute units end their tiles together, and 128 KB from each of them
+     * would wait for the write-back of as many dirty lines of the L2s (a launch without any store is a tenth shorter).  BF16, us:
+     * 30229 x 2048 -> 11264 1174 -> 1133, 27000 x 4096 -> 16896 3106 -> 2967 */
+    auto store_rows = [&](const auto &h, gd_elem *at, uint32_t step) __attribute__((always_inline)) {
+        constexpr uint32_t ROWS = sizeof(h) / sizeof(h[0]);
+        if (p.flags & GD_HIP_LINEAR_STREAM_Y) {
+            asm volatile("; streaming"); /* the compiler makes one ordinary store of two that differ in the hint alone */
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS; ++r) __builtin_nontemporal_store(h[r], reinterpret_cast<gd_elem8 *>(at + r * step));
+            asm volatile("; streamed");
+        } else {
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS; ++r) *reinterpret_cast<gd_elem8 *>(at + r * step) = h[r];
+        }
+    };
     auto epilogue_own = [&](auto mode_tag) __attribute__((always_inline)) {
         if (decltype(mode_tag)::value != GD_HIP_EPI_NONE) load_bias();
         unsigned char *own = epi + wave * 8192u;
@@ -721,8 +732,8 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
 #pragma unroll
                     for (int t = 0; t < 8; ++t) h[it][t] = res[it][t] + h[it][t];
                 }
-                store_own(h[it], ytile + ((uint32_t)I * 32u + it * 4u) * p.ldy + y_lane);
             }
+            store_rows(h, ytile + (uint32_t)I * 32u * p.ldy + y_lane, 4u * p.ldy);
         };
         pass(std::integral_constant<int, 0>{});
         pass(std::integral_constant<int, 1>{});
@@ -764,9 +775,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 const uint32_t e = it * 8u + rr;
                 h[it] = *reinterpret_cast<const gd_elem8 *>(own + (e * 8u + (v ^ ((e >> 1) & 7u))) * 16u);
             }
-#pragma unroll
-            for (uint32_t it = 0; it < 4u; ++it)
-                store_own(h[it], ytile + ((uint32_t)I * 32u + it * 8u) * p.ldy + y_lane);
+            store_rows(h, ytile + (uint32_t)I * 32u * p.ldy + y_lane, 8u * p.ldy);
         };
         pass(std::integral_constant<int, 0>{});
         pass(std::integral_constant<int, 1>{});
@@ -991,6 +1000,20 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
     }
 }
 
+/* Streaming stores for outputs of 64 MiB and more, twice the L2s: what reads a smaller one finds part of it there.  BF16, us, two
+ * projections, a gated one and a normalised residual addition behind them, with ordinary stores and with this rule (all stores
+ * streaming): 2048 rows of 2048 columns (outputs of 17, 23 and 8 MB) 232.5, 232.5 (247.5); 4096 x 1024 (17, 23, 8) 137.4, 137.4
+ * (145.1); 4096 x 2048 (34, 46, 17) 365.7, 365.3 (369.2); 4096 x 4096 (67, 92, 34) 1257, 1241 (1241); 16384 x 1024 (67, 92, 34) 470, 456
+ * (457); 16384 x 2048 (134, 185, 67) 1421, 1398 (1400); the exception is 8192 x 2048 (67, 92, 34) 717, 725 (726).  A reader of a
+ * larger output pays: the norms and rotations of 24,000 latent rows 31 -> 36 us. */
+#define GD_TILE_STREAM_BYTES (64u << 20)
+static inline gd_hip_linear_params gd_tile_streamed(const gd_hip_linear_params &params)
+{
+    gd_hip_linear_params p = params;
+    if ((uint64_t)p.M * p.N * 2u >= GD_TILE_STREAM_BYTES) p.flags |= GD_HIP_LINEAR_STREAM_Y;
+    return p;
+}
+
 #ifdef GD_LINEAR_TILE_GROUPED
 template <int WM, int WN>
 static int launch_tile_grouped(hipStream_t stream, const gd_elem *x, const gd_elem *w, gd_elem *y,
@@ -1024,9 +1047,10 @@ extern "C" int gd_hip_launch_linear_tile_grouped_bf16(hipStream_t stream, const 
 {
     const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
     const gd_tile_group group = {first, tiles, w_rows};
+    const gd_hip_linear_params s = gd_tile_streamed(*p);
     if (big_tiles)
-        return launch_tile_grouped<4, 4>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, *p, group, max_tiles, units);
-    return launch_tile_grouped<2, 2>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, *p, group, max_tiles, 2u * units);
+        return launch_tile_grouped<4, 4>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, s, group, max_tiles, units);
+    return launch_tile_grouped<2, 2>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, s, group, max_tiles, 2u * units);
 }
 #else
 template <int WM, int WN, bool W_NK, int PRO>
@@ -1109,7 +1133,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear_tile)(hipStream_t stream, const
                                          const gd_hip_linear_params *params, int big_tiles, int vector_store,
                                          int compute_units)
 {
-    const gd_hip_linear_params &p = *params;
+    const gd_hip_linear_params p = gd_tile_streamed(*params);
     const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
     const gd_elem *xp = (const gd_elem *)x, *rp = (const gd_elem *)residual;
     gd_elem *yp = (gd_elem *)y;

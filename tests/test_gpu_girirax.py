@@ -20,6 +20,13 @@ def arena(backend):
     backend.free(buf)
 
 
+@pytest.fixture()
+def large(backend):
+    buf = backend.buffer(512 << 20)
+    yield buf
+    backend.free(buf)
+
+
 @pytest.fixture(scope="module")
 def L():
     from oracle import layer_list
@@ -153,6 +160,33 @@ def test_a_gated_row_does_not_depend_on_its_tile(backend, gda, arena, kind):
     backend.fused_linear(x, w, b, None, None, whole, True, 1, 0, epilogue=kind)
     backend.fused_linear(x.rows(0, M), w, b, None, None, ragged, True, 1, 0, epilogue=kind)
     assert np.array_equal(whole.read()[:M], ragged.read())
+
+
+@pytest.mark.parametrize("dtype", [1, BF16], ids=["f16", "bf16"])
+def test_rows_of_large_outputs_are_those_of_small_ones(backend, gda, large, dtype):
+    """Outputs of 71 MB, which are stored past the caches, against the same rows in an output of 38 MB: plain, with a residual (F16)
+    and gated, whole tiles and a ragged last one."""
+    M, part, N, K = 4355, 2304, 8192, 128
+    rng = np.random.default_rng(dtype)
+    x, xv = _put(large, dtype, rng.standard_normal((M, K)))
+    w, wv = _put(large, dtype, rng.standard_normal((N, K)) / np.sqrt(K))
+    y, few = large.alloc((M, N), dtype), large.alloc((part, N), dtype)
+    for first in (0, M - part):
+        backend.matmul_nt(x, w, y)
+        backend.matmul_nt(x.rows(first, part), w, few)
+        assert np.array_equal(few.read(), y.read()[first:first + part])
+    picked = np.concatenate([np.arange(0, M, 173), [M - 1]])
+    _near(y.read_float()[picked], xv[picked] @ wv.T, dtype if dtype == BF16 else BF16)
+    if dtype == 1:
+        r, _ = _put(large, dtype, rng.standard_normal((1, N)).repeat(M, 0))
+        backend.fused_linear(x, w, None, r, None, y, True, 0, 0)
+        backend.fused_linear(x.rows(0, part), w, None, r.rows(0, part), None, few, True, 0, 0)
+        assert np.array_equal(few.read(), y.read()[:part])
+    top, half = large.alloc((2 * M, N // 2), dtype), large.alloc((part, N // 2), dtype)
+    twice, _ = _put(large, dtype, rng.standard_normal((2 * M, K)))
+    backend.fused_linear(twice, w, None, None, None, top, True, 0, 0, epilogue=1)
+    backend.fused_linear(twice.rows(300, part), w, None, None, None, half, True, 0, 0, epilogue=1)
+    assert np.array_equal(half.read(), top.read()[300:300 + part])
 
 
 # ---- residual stream --------------------------------------------------------------------------------------
