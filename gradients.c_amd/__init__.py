@@ -246,6 +246,7 @@ _SIGNATURES = {
     "gd_backend_set_tunable": [_vp, C.c_char_p, C.c_int64],
     "gd_backend_sdpa_decode_last_kernel": [_vp, C.c_char_p, C.c_size_t],
     "gd_backend_linear_last_kernel": [_vp, C.c_char_p, C.c_size_t],
+    "gd_backend_linear_last_form": [_vp, C.c_char_p, C.c_size_t],
 }
 _OTHER_RESTYPE = {
     "gd_backend_destroy": (None, [_vp]),
@@ -459,6 +460,11 @@ class Backend:
     def linear_last_kernel(self):
         out = C.create_string_buffer(32)
         _check(lib().gd_backend_linear_last_kernel(self.handle, out, 32), "gd_backend_linear_last_kernel")
+        return out.value.decode()
+
+    def linear_last_form(self):
+        out = C.create_string_buffer(32)
+        _check(lib().gd_backend_linear_last_form(self.handle, out, 32), "gd_backend_linear_last_form")
         return out.value.decode()
 
     def sdpa_decode_last_kernel(self):

@@ -368,7 +368,17 @@ gd_status gd_backend_linear_last_kernel(gd_backend *backend, char *out, size_t c
 {
     static const char *const names[] = {NULL, "stream", "wide", "tile", "scalar", "f32"};
     if (backend == NULL || out == NULL || capacity == 0u) return GD_ERR_INVALID_ARGUMENT;
-    if (backend->last_linear_family < 1 || backend->last_linear_family > 5) return GD_ERR_BAD_STATE;
-    snprintf(out, capacity, "%s", names[backend->last_linear_family]);
+    if (backend->last_linear_family < 1) return GD_ERR_BAD_STATE;
+    snprintf(out, capacity, "%s", names[backend->last_linear_family & 255]);
+    return GD_OK;
+}
+
+/* Which form of the "wide" family the last projection call took: "tile", "persistent" or "half"; "" for other families. */
+gd_status gd_backend_linear_last_form(gd_backend *backend, char *out, size_t capacity)
+{
+    static const char *const names[] = {"", "tile", "persistent", "half"};
+    if (backend == NULL || out == NULL || capacity == 0u) return GD_ERR_INVALID_ARGUMENT;
+    if (backend->last_linear_family < 1) return GD_ERR_BAD_STATE;
+    snprintf(out, capacity, "%s", names[backend->last_linear_family >> 8]);
     return GD_OK;
 }

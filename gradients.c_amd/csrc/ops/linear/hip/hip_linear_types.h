@@ -60,6 +60,11 @@ _Static_assert(sizeof(gd_hip_linear_params) == 76, "the few-row kernel's argumen
 #define GD_HIP_LINEAR_FAMILY_SCALAR 4 /* unaligned operands */
 #define GD_HIP_LINEAR_FAMILY_F32 5    /* F32 operands (linear_f32.hip) */
 
+/* form of the wide family: what gd_hip_try_launch_linear_wide returns */
+#define GD_HIP_LINEAR_WIDE_TILE 1       /* a column tile per workgroup */
+#define GD_HIP_LINEAR_WIDE_PERSISTENT 2 /* runs of column tiles */
+#define GD_HIP_LINEAR_WIDE_HALF 3       /* 8 columns per workgroup */
+
 /* destinations of the rope + append epilogue: q [M,H,D]; caches [M,Tmax,H,D]; positions I32 [M] */
 typedef struct gd_hip_rope_epilogue {
     const int32_t *rope_pos, *cache_pos;

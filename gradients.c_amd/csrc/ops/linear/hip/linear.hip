@@ -145,7 +145,9 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear)(hipStream_t stream, const void
                                     int store_vector_ok, int min_workgroups, const gd_hip_rope_epilogue *rope_epilogue,
                                     int wide_mode, int *family)
 {
-    /* *family: which kernel family took the call (GD_HIP_LINEAR_FAMILY_*), for logs and tests */
+    /* *family: which kernel family took the call (GD_HIP_LINEAR_FAMILY_*; GD_HIP_LINEAR_WIDE_* * 256 with the wide one), for logs
+     * and tests */
+    int form = 0;
     *family = GD_HIP_LINEAR_FAMILY_STREAM;
     const gd_hip_rope_epilogue no_rope = {nullptr, nullptr, nullptr, nullptr, nullptr};
     const gd_hip_rope_epilogue &rope = rope_epilogue != nullptr ? *rope_epilogue : no_rope;
@@ -184,13 +186,13 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear)(hipStream_t stream, const void
 #endif
         return GD_LINEAR_FN(gd_hip_launch_linear_tile)(stream, x, w, bias, residual, norm_w, y, params, big >= units, store_vector_ok, (int)units);
     } else if (wide_mode != 0 && p.w_is_nk &&
-               GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(stream, x, w, bias, residual, norm_w, y, params, rope_epilogue,
-                                             wide_mode > 0 ? 0u : (4ull << 20), p.force_tiles,
-                                             min_workgroups > 0 ? (uint32_t)min_workgroups / 2u : 256u)) {
+               (form = GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(stream, x, w, bias, residual, norm_w, y, params, rope_epilogue,
+                                                     wide_mode > 0 ? 0u : (4ull << 20), p.force_tiles,
+                                                     min_workgroups > 0 ? (uint32_t)min_workgroups / 2u : 256u)) != 0) {
         /* weight matrices of megabytes: the kernel built around the weight stream (wide_mode: 0 never, 1 whenever it
          * covers the call, -1 from 4 MiB of weights on; below that the launch latency decides and the stream kernel
          * is shorter) */
-        *family = GD_HIP_LINEAR_FAMILY_WIDE;
+        *family = GD_HIP_LINEAR_FAMILY_WIDE + 256 * form;
     } else {
         /* columns per workgroup: 64, 32 or 16 (rows: always 16, further rows in grid.y; their weight re-reads
          * come from L2).  More columns reuse each activation fragment for more MFMAs and repeat the prologue

@@ -88,7 +88,7 @@ static bool launch_persistent_rows(hipStream_t stream, const void *x, const void
 }
 #endif
 
-/* Returns 1 when the launch was taken (hipGetLastError() then tells how it went), 0 when this kernel family does
+/* Returns the form (GD_HIP_LINEAR_WIDE_*) that took the launch (hipGetLastError() then tells how it went), 0 when this kernel family does
  * not cover the call and the caller goes on to the stream kernel.  Covered: [N,K] weights of at least min_bytes
  * whose K is a multiple of 64 and splits over the eight wavefronts into at most 4 (behind an rms_norm) or 12 (no
  * prologue) pairs of steps each, fewer than 128 rows, and
@@ -114,7 +114,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
 #if GD_LINEAR_IS_BF16
     /* K that the eight wavefronts share in whole pairs of steps: the persistent form; other K and narrower outputs go on */
     if (tiles != 1u && p.prologue == GD_HIP_PRO_NONE && epi != GD_WIDE_EPI_ROPE) {
-#define GD_R(PMAX, EPI) if (p.K == 512u * PMAX && launch_persistent_rows<PMAX, EPI>(stream, x, w, bias, y, p, rope, units)) return 1
+#define GD_R(PMAX, EPI) if (p.K == 512u * PMAX && launch_persistent_rows<PMAX, EPI>(stream, x, w, bias, y, p, rope, units)) return GD_HIP_LINEAR_WIDE_PERSISTENT
         if (epi == GD_WIDE_EPI_PLAIN) {
             GD_R(1, GD_WIDE_EPI_PLAIN);
             GD_R(2, GD_WIDE_EPI_PLAIN);
@@ -130,7 +130,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
 #endif
     const bool persistent = tiles != 1u; /* "linear_tiles" = 1 asks for the one-tile-per-workgroup form (for comparison) */
 #define GD_W(NT, MT, PMAX, PRO, EPI) \
-    do { launch_wide<NT, MT, PMAX, PRO, EPI>(stream, x, w, bias, residual, norm_w, y, p, rope); return 1; } while (0)
+    do { launch_wide<NT, MT, PMAX, PRO, EPI>(stream, x, w, bias, residual, norm_w, y, p, rope); return GD_HIP_LINEAR_WIDE_TILE; } while (0)
 #define GD_W_MT(NT, PMAX, PRO, EPI) \
     do { if (mt == 1u) GD_W(NT, 1, PMAX, PRO, EPI); if (mt == 2u) GD_W(NT, 2, PMAX, PRO, EPI); GD_W(NT, 4, PMAX, PRO, EPI); } while (0)
     if (p.prologue == GD_HIP_PRO_NONE && epi == GD_WIDE_EPI_PLAIN && (p.N % 16u) == 0u) {
@@ -141,12 +141,12 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
          * streams (16 x 5632 -> 2048: 256 workgroups instead of 128) */
         if (p.M <= 16u && p.N / 16u < units && tiles != 1u && (p.K % 128u) == 0u && (p.N % 8u) == 0u) {
             const uint32_t qpw = (p.K / 128u + 7u) / 8u; /* pieces of 128 per wavefront */
-            if (qpw <= 2u) { launch_wide_half<2>(stream, x, w, bias, residual, y, p); return 1; }
-            if (qpw <= 6u) { launch_wide_half<6>(stream, x, w, bias, residual, y, p); return 1; }
+            if (qpw <= 2u) { launch_wide_half<2>(stream, x, w, bias, residual, y, p); return GD_HIP_LINEAR_WIDE_HALF; }
+            if (qpw <= 6u) { launch_wide_half<6>(stream, x, w, bias, residual, y, p); return GD_HIP_LINEAR_WIDE_HALF; }
 #if GD_LINEAR_IS_BF16
             /* (8448 -> 2048 at 4 and 16 rows: 12.7 and 17.0 us, the stream kernel's four wavefronts 14.7 and 18.3; what is left is the
              * activation matrix, which every 8 columns read whole) */
-            if (qpw <= 12u) { launch_wide_half<12>(stream, x, w, bias, residual, y, p); return 1; }
+            if (qpw <= 12u) { launch_wide_half<12>(stream, x, w, bias, residual, y, p); return GD_HIP_LINEAR_WIDE_HALF; }
 #endif
         }
         if (ppw <= 4u) GD_W(1, 1, 4, GD_HIP_PRO_NONE, GD_WIDE_EPI_PLAIN);
@@ -160,7 +160,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
     if (p.prologue != GD_HIP_PRO_RMS_NORM || ppw > 4u) return 0;
     /* K = 2048: the persistent form, where its LDS holds the sums of MT x NT tiles next to the ring */
 #define GD_P(NT, MT, EPI) \
-    do { launch_persistent<NT, MT, 4, EPI, GD_HIP_PRO_RMS_NORM>(stream, x, w, bias, residual, norm_w, y, p, rope, units, tiles != 4u, 0u); return 1; } while (0)
+    do { launch_persistent<NT, MT, 4, EPI, GD_HIP_PRO_RMS_NORM>(stream, x, w, bias, residual, norm_w, y, p, rope, units, tiles != 4u, 0u); return GD_HIP_LINEAR_WIDE_PERSISTENT; } while (0)
     if (p.K == 2048u && persistent) {
         if (epi == GD_WIDE_EPI_PLAIN && (p.N % 64u) == 0u && mt <= 2u) {
             if (mt == 1u) GD_P(4, 1, GD_WIDE_EPI_PLAIN);

@@ -30,6 +30,7 @@ GD_NULL_OP(gd_backend_kv_cache_append_positions)
 GD_NULL_OP(gd_backend_latent_attend)
 GD_NULL_OP(gd_backend_latent_prepare)
 GD_NULL_OP(gd_backend_linear)
+GD_NULL_OP(gd_backend_linear_last_form)
 GD_NULL_OP(gd_backend_linear_last_kernel)
 GD_NULL_OP(gd_backend_linear_nt)
 GD_NULL_OP(gd_backend_linear_qkv_rope_packed)

@@ -121,6 +121,46 @@ def test_few_rows_onto_many_columns(backend, gda, arena, M, N, K):
     _near(half.read_float(), (want + bv)[:, :N] * gate / (1 + np.exp(-gate)), BF16)
 
 
+def _few_rows(backend, arena, M, N, K, plain, gated):
+    """N plain outputs, to BF16 and F32, or N gated ones, and the form of the wide family that has to take them."""
+    rng = np.random.default_rng(M + N + K)
+    x, xv = _put(arena, BF16, rng.standard_normal((M, K)))
+    rows = N if gated is None else 2 * N
+    w, wv = _put(arena, BF16, rng.standard_normal((rows, K), np.float32) / np.sqrt(K))
+    b, bv = _put(arena, BF16, rng.standard_normal(rows))
+    want = xv @ wv.T
+    if gated is None:
+        y, wide = arena.alloc((M, N), BF16), arena.alloc((M, N), F32)
+        backend.fused_linear(x, w, b, None, None, y, True, 1, 0)
+        assert backend.linear_last_form() == plain
+        _near(y.read_float(), want + bv, BF16)
+        backend.matmul_nt(x, w, wide)
+        assert backend.linear_last_form() == plain
+        _near(wide.read_float(), want, F32, factor=3)
+    else:
+        half, gate = arena.alloc((M, N), BF16), (want + bv)[:, N:]
+        backend.fused_linear(x, w, b, None, None, half, True, 1, 0, epilogue=1)
+        assert backend.linear_last_form() == gated
+        _near(half.read_float(), (want + bv)[:, :N] * gate / (1 + np.exp(-gate)), BF16)
+
+
+#: columns of 192 workgroups (three quarters of the compute units), a few more, and the last tile not full
+@pytest.mark.parametrize("M,N,K", [(4, 12250, 2048), (20, 12250, 2048), (64, 6150, 2048), (100, 6150, 2048), (17, 12250, 4096), (33, 6150, 4096),
+                                   (64, 12250, 4096), (1, 6150, 4096), (16, 12300, 1024), (33, 6150, 512)])
+def test_persistent_forms_of_few_rows(backend, gda, arena, M, N, K):
+    """One, two and four row tiles over 64 and 32 columns per tile, plain; gated with half as many outputs."""
+    _few_rows(backend, arena, M, N, K, "persistent", None)
+    if K > 512:
+        _few_rows(backend, arena, M, N // 2, K, None, "persistent")
+
+
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("N,K", [(1024, 6272), (1040, 8320), (2048, 8448), (528, 12288)])
+def test_eight_columns_of_long_rows(backend, gda, arena, M, N, K):
+    """More pieces of K per wavefront than the ring holds, the same number for all wavefronts and not."""
+    _few_rows(backend, arena, M, N, K, "half", None)
+
+
 def test_big_tiles_and_unsupported_forms(backend, gda, arena):
     """Enough 256 x 256 tiles for every compute unit, with ragged edges, plain and gated; and what BF16 does not have."""
     rng = np.random.default_rng(5)
