@@ -72,7 +72,12 @@ static bool launch_persistent(hipStream_t stream, const void *x, const void *w, 
  *   1024 -> 32768 F32 results  15.5, 15.9, 18.1, 22.2 (24.7, 29.1, 53.1, 99.9): 4.3 to 3.0 TB/s
  *   2048 -> 32768 F32 results  30.1, 29.6, 31.8, 37.2 (37.1, 38.6, 67.3, 121): 4.5 to 3.6 TB/s
  *   1024 -> 2816 gated         5.1, 5.1, 6.1, 8.7 (5.9, 6.4, 8.6, 14.3);  2048 -> 5632 gated 12.2, 12.8, 14.9, 21.0 (15.9, 16.5, 26.3, 37.1)
- *   1024 -> 4384               4.6, 4.8, 5.8, 8.3 (6.6, 7.7, 11.0, 17.5);  4096 -> 8448 17.5, 19.1, 22.8, 41.0 (24.1, 31.0, 48.3, 82.8) */
+ *   1024 -> 4384               4.6, 4.8, 5.8, 8.3 (6.6, 7.7, 11.0, 17.5);  4096 -> 8448 17.5, 19.1, 22.8, 41.0 (24.1, 31.0, 48.3, 82.8)
+ * and for the K between the powers of two (us; 1, 16, 32, 64 rows):
+ *   1536 -> 32768 F32 results  21.7, 22.4, 24.6, 29.3 (26.8, 34.3, 60.2, 112);  3072 -> 32768 41.7, 40.8, 44.3, 77.2 (48.7, 73.5, 135, 257)
+ *   1536 -> 6144               6.2, 7.1, 8.3, 11.6 (7.6, 9.6, 13.0, 22.6);  2560 -> 6144 8.6, 10.0, 12.6, 21.0 (12.5, 18.6, 26.1, 48.7)
+ *   512 -> 8448 gated          7.5, 8.1, 9.4, 11.4 (8.4, 9.0, 11.2, 15.6);  1536 -> 4224 gated 8.4, 9.3, 10.9, 15.8 (11.3, 12.5, 20.8, 30.1)
+ *   3072 -> 8448 gated         29.0, 30.5, 34.6, 58.7 (37.7, 41.0, 55.5, 85.8);  3584 -> 3072 gated 11.3, 12.8, 16.3, 28.1 (12.8, 15.1, 22.9, 38.9) */
 template <int PMAX, int EPI>
 static bool launch_persistent_rows(hipStream_t stream, const void *x, const void *w, const void *bias, void *y,
                                    const gd_hip_linear_params &p, const gd_hip_rope_epilogue &rope, uint32_t units)
@@ -88,14 +93,16 @@ static bool launch_persistent_rows(hipStream_t stream, const void *x, const void
 }
 #endif
 
-/* Returns the form (GD_HIP_LINEAR_WIDE_*) that took the launch (hipGetLastError() then tells how it went), 0 when this kernel family does
- * not cover the call and the caller goes on to the stream kernel.  Covered: [N,K] weights of at least min_bytes
- * whose K is a multiple of 64 and splits over the eight wavefronts into at most 4 (behind an rms_norm) or 12 (no
- * prologue) pairs of steps each, fewer than 128 rows, and
- *   plain epilogue:   no prologue, 16 columns per workgroup (8 where that leaves compute units without one);
- *                     rms_norm prologue, 64 columns per workgroup;
- *   swiglu epilogue:  rms_norm prologue, 32 (tiles == 2) or 64 weight rows per workgroup;
- *   rope epilogue:    rms_norm prologue, 32 weight rows per workgroup (head size a multiple of 32). */
+/* Returns the form (GD_HIP_LINEAR_WIDE_*) that took the launch (hipGetLastError() then tells how it went), 0 when this
+ * kernel family does not cover the call and the caller goes on to the stream kernel.  Covered: [N,K] weights of at least
+ * min_bytes whose K is a multiple of 64, fewer than 128 rows, and
+ *   BF16, K = 512 to 4096 in steps of 512, column tiles for three quarters of the compute units: plain and gated in the
+ *                     persistent form (launch_persistent_rows);
+ *   plain epilogue:   no prologue, 16 columns per workgroup (8 where that leaves compute units without one), K that splits
+ *                     over the eight wavefronts into at most 12 pairs of steps each; F16 behind an rms_norm, at most 4
+ *                     pairs, 64 columns per workgroup;
+ *   swiglu epilogue:  F16 behind an rms_norm, 32 (tiles == 2) or 64 weight rows per workgroup;
+ *   rope epilogue:    F16 behind an rms_norm, 32 weight rows per workgroup (head size a multiple of 32). */
 extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, const void *x, const void *w, const void *bias,
                                              const void *residual, const void *norm_w, void *y,
                                              const gd_hip_linear_params *params, const gd_hip_rope_epilogue *rope_epilogue,
@@ -112,18 +119,17 @@ extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_wide)(hipStream_t stream, c
     const int epi = p.rope_head_dim != 0u ? GD_WIDE_EPI_ROPE : (p.swiglu_cols != 0u ? GD_WIDE_EPI_SWIGLU : GD_WIDE_EPI_PLAIN);
     const uint32_t mt = p.M <= 16u ? 1u : (p.M <= 32u ? 2u : 4u);
 #if GD_LINEAR_IS_BF16
-    /* K that the eight wavefronts share in whole pairs of steps: the persistent form; other K and narrower outputs go on */
-    if (tiles != 1u && p.prologue == GD_HIP_PRO_NONE && epi != GD_WIDE_EPI_ROPE) {
-#define GD_R(PMAX, EPI) if (p.K == 512u * PMAX && launch_persistent_rows<PMAX, EPI>(stream, x, w, bias, y, p, rope, units)) return GD_HIP_LINEAR_WIDE_PERSISTENT
-        if (epi == GD_WIDE_EPI_PLAIN) {
-            GD_R(1, GD_WIDE_EPI_PLAIN);
-            GD_R(2, GD_WIDE_EPI_PLAIN);
-            GD_R(4, GD_WIDE_EPI_PLAIN);
-            GD_R(8, GD_WIDE_EPI_PLAIN);
-        } else {
-            GD_R(2, GD_WIDE_EPI_SWIGLU);
-            GD_R(4, GD_WIDE_EPI_SWIGLU);
-            GD_R(8, GD_WIDE_EPI_SWIGLU);
+    /* K that the eight wavefronts share in whole pairs of steps, up to the pairs whose activations fit a lane's registers: the
+     * persistent form; other K and narrower outputs go on */
+    if (tiles != 1u && p.prologue == GD_HIP_PRO_NONE && epi != GD_WIDE_EPI_ROPE && (p.K % 512u) == 0u) {
+#define GD_R(PMAX)                                                                                                           \
+    case PMAX:                                                                                                              \
+        if (epi == GD_WIDE_EPI_PLAIN ? launch_persistent_rows<PMAX, GD_WIDE_EPI_PLAIN>(stream, x, w, bias, y, p, rope, units) \
+                                     : launch_persistent_rows<PMAX, GD_WIDE_EPI_SWIGLU>(stream, x, w, bias, y, p, rope, units)) \
+            return GD_HIP_LINEAR_WIDE_PERSISTENT;                                                                           \
+        break
+        switch (p.K / 512u) {
+            GD_R(1); GD_R(2); GD_R(3); GD_R(4); GD_R(5); GD_R(6); GD_R(7); GD_R(8);
         }
 #undef GD_R
     }

@@ -146,12 +146,12 @@ def _few_rows(backend, arena, M, N, K, plain, gated):
 
 #: columns of 192 workgroups (three quarters of the compute units), a few more, and the last tile not full
 @pytest.mark.parametrize("M,N,K", [(4, 12250, 2048), (20, 12250, 2048), (64, 6150, 2048), (100, 6150, 2048), (17, 12250, 4096), (33, 6150, 4096),
-                                   (64, 12250, 4096), (1, 6150, 4096), (16, 12300, 1024), (33, 6150, 512)])
+                                   (64, 12250, 4096), (1, 6150, 4096), (16, 12300, 1024), (33, 6150, 512),
+                                   (3, 12250, 1536), (64, 6150, 1536), (18, 6150, 2560), (16, 6150, 3072), (47, 6200, 3072), (40, 12250, 3584)])
 def test_persistent_forms_of_few_rows(backend, gda, arena, M, N, K):
     """One, two and four row tiles over 64 and 32 columns per tile, plain; gated with half as many outputs."""
     _few_rows(backend, arena, M, N, K, "persistent", None)
-    if K > 512:
-        _few_rows(backend, arena, M, N // 2, K, None, "persistent")
+    _few_rows(backend, arena, M, max(N // 2, (4 << 20) // (2 * K)), K, None, "persistent")
 
 
 @pytest.mark.parametrize("M", [1, 16])
