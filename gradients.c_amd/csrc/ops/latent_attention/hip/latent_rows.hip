@@ -292,9 +292,12 @@ gd_latent_value_kernel(const float *__restrict__ o_lat, const T *__restrict__ w_
     }
 }
 
-/* four rows to a workgroup where that leaves two workgroups for every compute unit of the chip (six portions of 160 to 570 rows, 8 heads,
+/* four rows to a workgroup where that leaves two workgroups for every compute unit (six portions of 160 to 570 rows, 8 heads,
  * three of them shared, mean: value 67 -> 33, query 41 -> 24 us), one otherwise, so that every unit has work */
-static bool gd_latent_rows_share(uint32_t rows, uint32_t heads) { return (uint64_t)rows * heads >= 4u * 512u; }
+static bool gd_latent_rows_share(uint32_t rows, uint32_t heads, uint32_t units)
+{
+    return (uint64_t)rows * heads >= 4u * 2u * (uint64_t)units;
+}
 
 extern "C" int gd_hip_launch_latent_prepare(hipStream_t stream, const void *proj, uint32_t ld, const float *q_norm,
                                             const float *kv_norm, const float *freq, float *angles, void *cq, void *cache,
@@ -314,10 +317,11 @@ extern "C" int gd_hip_launch_latent_prepare(hipStream_t stream, const void *proj
 }
 
 extern "C" int gd_hip_launch_latent_query(hipStream_t stream, const void *qv, const void *w_ukt, const float *angles,
-                                          void *ql, const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32)
+                                          void *ql, const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32,
+                                          uint32_t units)
 {
 #define GD_GO(T, R) gd_latent_query_kernel<T, R><<<dim3((q->rows + R - 1u) / R, m->heads), 256, R * m->dim * sizeof(float), stream>>>((const T *)qv, (const T *)w_ukt, angles, (T *)ql, *m, q->rows)
-    if (gd_latent_rows_share(q->rows, m->heads) && m->dim <= 2048u) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
+    if (gd_latent_rows_share(q->rows, m->heads, units) && m->dim <= 2048u) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
     else { if (is_f32) GD_GO(float, 1); else GD_GO(gd_bf16, 1); }
 #undef GD_GO
     return (int)hipGetLastError();
@@ -337,11 +341,12 @@ extern "C" int gd_hip_launch_latent_attend(hipStream_t stream, const void *ql, c
 }
 
 extern "C" int gd_hip_launch_latent_value(hipStream_t stream, const float *o_lat, const void *w_uv, const void *gate,
-                                          uint32_t ldg, void *out, uint32_t rows, const gd_hip_latent_params *m, int is_f32)
+                                          uint32_t ldg, void *out, uint32_t rows, const gd_hip_latent_params *m, int is_f32,
+                                          uint32_t units)
 {
     if (rows == 0u) return (int)hipSuccess;
 #define GD_GO(T, R) gd_latent_value_kernel<T, R><<<dim3((rows + R - 1u) / R, m->heads), 256, R * m->kv_rank * sizeof(float), stream>>>(o_lat, (const T *)w_uv, (const T *)gate, ldg, (T *)out, *m, rows)
-    if (gd_latent_rows_share(rows, m->heads)) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
+    if (gd_latent_rows_share(rows, m->heads, units)) { if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4); }
     else { if (is_f32) GD_GO(float, 1); else GD_GO(gd_bf16, 1); }
 #undef GD_GO
     return (int)hipGetLastError();

@@ -95,7 +95,8 @@ static bool launch_persistent_rows(hipStream_t stream, const void *x, const void
 
 /* Returns the form (GD_HIP_LINEAR_WIDE_*) that took the launch (hipGetLastError() then tells how it went), 0 when this
  * kernel family does not cover the call and the caller goes on to the stream kernel.  Covered: [N,K] weights of at least
- * min_bytes whose K is a multiple of 64, fewer than 128 rows, and
+ * min_bytes and below 2^29 elements (byte offsets of both sections of a paired weight in 31 bits; plain weights beyond that,
+ * 131,072 x 4096, take the stream kernel) whose K is a multiple of 64, fewer than 128 rows, and
  *   BF16, K = 512 to 4096 in steps of 512, column tiles for three quarters of the compute units: plain and gated in the
  *                     persistent form (launch_persistent_rows);
  *   plain epilogue:   no prologue, 16 columns per workgroup (8 where that leaves compute units without one), K that splits
