@@ -1000,17 +1000,19 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
     }
 }
 
-/* Streaming stores for outputs of 64 MiB and more, twice the L2s: what reads a smaller one finds part of it there.  BF16, us, two
- * projections, a gated one and a normalised residual addition behind them, with ordinary stores and with this rule (all stores
- * streaming): 2048 rows of 2048 columns (outputs of 17, 23 and 8 MB) 232.5, 232.5 (247.5); 4096 x 1024 (17, 23, 8) 137.4, 137.4
- * (145.1); 4096 x 2048 (34, 46, 17) 365.7, 365.3 (369.2); 4096 x 4096 (67, 92, 34) 1257, 1241 (1241); 16384 x 1024 (67, 92, 34) 470, 456
- * (457); 16384 x 2048 (134, 185, 67) 1421, 1398 (1400); the exception is 8192 x 2048 (67, 92, 34) 717, 725 (726).  A reader of a
- * larger output pays: the norms and rotations of 24,000 latent rows 31 -> 36 us. */
-#define GD_TILE_STREAM_BYTES (64u << 20)
+/* Streaming stores for outputs larger than the L2s together: what reads a smaller one finds part of it there.  Two projections, a
+ * gated one and a normalised residual addition behind them, BF16, us, with ordinary and with streaming stores: 2048 rows of 2048
+ * columns (outputs of 17, 23 and 8 MB) 232.5 (247.5), 4096 x 1024 (17, 23, 8) 137.4 (145.1); 16384 x 1024 (67, 92, 34) 470 (457),
+ * 16384 x 2048 (134, 185, 67) 1421 (1400).  Where the line lies between, whole prefills with all stores streaming, and streaming
+ * beyond 32 and from 64 MiB on: 18,000 rows of a 512-column F16 decoder (outputs of 19 to 57 MB) 2109, 2107, 2122; 12,500 rows
+ * 878, 879, 887; the BF16 layers of 2048 columns, 3,500 rows (14 to 60 MB) 3828, 3825, 3810; 13,600 rows of 1024 columns
+ * 6734, 6737, 6713; others differ by less.  A reader of a larger output pays: the norms and rotations of 24,000 latent rows 31 ->
+ * 36 us. */
+#define GD_TILE_STREAM_BYTES (32u << 20)
 static inline gd_hip_linear_params gd_tile_streamed(const gd_hip_linear_params &params)
 {
     gd_hip_linear_params p = params;
-    if ((uint64_t)p.M * p.N * 2u >= GD_TILE_STREAM_BYTES) p.flags |= GD_HIP_LINEAR_STREAM_Y;
+    if ((uint64_t)p.M * p.N * 2u > GD_TILE_STREAM_BYTES) p.flags |= GD_HIP_LINEAR_STREAM_Y;
     return p;
 }
 
