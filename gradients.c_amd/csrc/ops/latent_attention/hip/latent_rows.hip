@@ -52,7 +52,7 @@ gd_latent_prepare_kernel(const T *__restrict__ proj, uint32_t ld, const float *_
 
 /* prepare for BF16 rows of q_rank + kv_rank <= 4096 in 16-byte pieces: a wavefront per row, the row in registers; bound by its
  * round trips, so everything the row needs is requested in front of the sums (64 rows of 512 + 256, a workgroup each: 6.5 -> 5.2
- * us; 24,000 rows: 36 us either way) */
+ * us; 24,000 rows: 36 us either way behind a projection that stores past the L2s, 31 behind one that does not) */
 __global__ void __launch_bounds__(256)
 gd_latent_prepare_vec_kernel(const gd_bf16 *__restrict__ proj, uint32_t ld, const float *__restrict__ q_norm,
                              const float *__restrict__ kv_norm, const float *__restrict__ freq, float *__restrict__ angles,

@@ -131,9 +131,10 @@ gd_status gd_gpt_decoder_extend(gd_gpt_decoder *dec, const int32_t *slots, int32
  *                                   (gd_backend_fused_linear, gd_backend_qkv_rope_append: 5 launches
  *                                   per layer), which keep every rounding point of the separate
  *                                   operators;
- *   GD_GPT_RESIDENT_KEEP_LOGITS     every step also copies its logits [batch, vocab] into the decoder's
- *                                   "last_logits" tensor (one more launch per step; greedy sessions only):
- *                                   after sync it holds the logits of the last step run. */
+ *   GD_GPT_RESIDENT_KEEP_LOGITS     every step leaves its logits [batch, vocab] in the decoder's "last_logits"
+ *                                   tensor (greedy sessions only): after sync it holds the logits of the
+ *                                   last step run.  The LM head writes them there by itself; behind
+ *                                   GD_GPT_RESIDENT_UNFUSED they are copied, one more launch per step. */
 #define GD_GPT_RESIDENT_HOLD_POSITIONS 1
 #define GD_GPT_RESIDENT_UNFUSED 2
 #define GD_GPT_RESIDENT_KEEP_LOGITS 4
