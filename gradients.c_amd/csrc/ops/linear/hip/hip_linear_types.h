@@ -56,7 +56,7 @@ _Static_assert(sizeof(gd_hip_linear_params) == 76, "the few-row kernel's argumen
 /* kernel family that took a projection call */
 #define GD_HIP_LINEAR_FAMILY_STREAM 1 /* few rows, MFMA fragments from global memory (linear_stream_kernel.h) */
 #define GD_HIP_LINEAR_FAMILY_WIDE 2   /* few rows, whole-line weight stream through an LDS ring (linear_wide_kernel.h) */
-#define GD_HIP_LINEAR_FAMILY_TILE 3   /* 128 rows and more, LDS-tiled MFMA kernel (linear_tile.hip) */
+#define GD_HIP_LINEAR_FAMILY_TILE 3   /* 128 rows and more, LDS-tiled MFMA kernels (linear_tile.hip, linear_tile_nk.hip) */
 #define GD_HIP_LINEAR_FAMILY_SCALAR 4 /* unaligned operands */
 #define GD_HIP_LINEAR_FAMILY_F32 5    /* F32 operands (linear_f32.hip) */
 

@@ -1,6 +1,6 @@
 /*
  * Element type of the projection kernels.  The kernels are written over gd_elem; a translation unit that defines
- * GD_LINEAR_BF16 before including them (linear_bf16.hip, linear_tile_bf16.hip, linear_wide_bf16.hip) gets BF16
+ * GD_LINEAR_BF16 before including them (linear_bf16.hip, linear_tile_bf16.hip, linear_tile_nk_bf16.hip, linear_wide_bf16.hip) gets BF16
  * operands, every other one F16.  The matrix instructions of the two types have the same shape, rate and operand
  * layout, so nothing else differs, except that the BF16 build
  *   - instantiates only what its callers use: [N,K] weights, no prologue, no rotation epilogue;

@@ -3,7 +3,9 @@
  *
  * Same contract and rounding points as the weight-streaming kernel in linear.hip (reference GEMMs
  * src/ops/_shared/gemm/metal_gemm_common.h:54-135 and :161-237); this one is for M >= 128 where the
- * work is bound by the matrix cores, not by weight traffic.
+ * work is bound by the matrix cores, not by weight traffic.  [N,K] weights without a prologue, whose
+ * outputs take 16-byte stores, go through the kernel of linear_tile_nk.hip instead, which this file's
+ * launcher asks first; here are [K,N] weights, prologues and unaligned outputs.
  *
  * Tiling.  A workgroup of 4 wavefronts (2 x 2) owns a BM x BN output tile, BM = BN = 256 or 128; a
  * wavefront owns (BM/2) x (BN/2) as WM x WN tiles of v_mfma_f32_32x32x16_f16 (4 x 4 tiles = 256
@@ -46,42 +48,10 @@
 #include "../../_shared/hip_device.h"
 #include "hip_linear_types.h"
 #include "linear_elem.h"
-#include "../../qkv_split_rope/hip/rope_device.h"
+#include "linear_tile_nk.h"
 #include <type_traits>
 
 #define GD_TILE_BK 64u
-
-/* Profiling build (make TILE_TIMELINE=1): the first wavefront of every workgroup notes, for its first 32 tiles, the
- * 100 MHz real-time counter at the start of the tile, after the K loop and after the epilogue, and the shader clock
- * ticks the K loop took (their ratio is the clock the chip ran at).  gd_hip_linear_tile_timeline copies the notes of
- * the last launch out; bench.py --probe tile_timeline prints them.  Not part of a normal build. */
-#ifdef GD_TILE_TIMELINE
-__device__ unsigned long long gd_tile_timeline[256 * 32 * 4];
-extern "C" __attribute__((visibility("default"))) int gd_hip_linear_tile_timeline(unsigned long long *host)
-{
-    return (int)hipMemcpyFromSymbol(host, HIP_SYMBOL(gd_tile_timeline), sizeof(gd_tile_timeline));
-}
-#define GD_TILE_NOTE(slot, value)                                                                              \
-    do {                                                                                                        \
-        if (threadIdx.x == 0 && blockIdx.x < 256u && timeline_tile < 32u)                                       \
-            gd_tile_timeline[(blockIdx.x * 32u + timeline_tile) * 4u + (slot)] = (value);                       \
-    } while (0)
-#else
-#define GD_TILE_NOTE(slot, value) do { } while (0)
-#endif
-
-/* Rotation + cache append epilogue of the packed prefill's qkv projection (ROPE instantiation): the tile kernel
- * writes rotated q rows to q [M, hd], rotated k rows and v rows into cache row cache_row[m] of the K / V caches
- * (row pitch hd), and no [M, 3*hd] intermediate.  cos / sin hold, F32, the angles of row m's position for the half_d
- * pairs of a head (NeoX pairing: column c of a head with column c + half_d) in the layout of the table kernel
- * (gd_rope_table_at in ops/qkv_split_rope/hip/qkv_split_rope.hip). */
-struct gd_tile_rope {
-    const float *cos, *sin;
-    const int32_t *cache_row; /* [M]; negative: the row's k and v go nowhere */
-    gd_elem *q, *k_cache, *v_cache;
-    uint32_t hd;     /* heads * head_dim, a multiple of 256 */
-    uint32_t half_d; /* 32 or 64 */
-};
 
 __device__ __forceinline__ uint32_t gd_tile_slot(uint32_t row, uint32_t c)
 {
@@ -124,24 +94,13 @@ __device__ __forceinline__ void gd_tile_load_lds16(const gd_elem *uniform_base, 
                  : "memory");
 }
 
-/* GROUPED instantiation: the rows are packed by group (the experts of a routed feed-forward), and every group has its own
- * weights, one behind the other.  tiles [0]: number of row tiles, then from [2] on (group, first row) of each, BM rows or
- * up to the group's end first[group + 1].  x rows behind the last group's are read and must exist (up to BM - 1). */
-struct gd_tile_group {
-    const int32_t *first, *tiles;
-    uint32_t w_rows; /* weight rows of a group */
-};
-__device__ __forceinline__ const gd_tile_rope &gd_tile_rope_of(const gd_tile_rope &r) { return r; }
-__device__ __forceinline__ gd_tile_rope gd_tile_rope_of(const gd_tile_group &) { return gd_tile_rope{}; }
-
-template <int WM, int WN, bool W_NK, int PRO, bool ROPE = false, bool GROUPED = false>
+template <int WM, int WN, bool W_NK, int PRO>
 __global__ void __launch_bounds__(256)
 gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__ w, const gd_elem *__restrict__ bias,
                       const gd_elem *__restrict__ residual, const gd_elem *__restrict__ norm_w,
                       gd_elem *__restrict__ y, gd_hip_linear_params p, uint32_t tiles_m, uint32_t tiles_n,
-                      uint32_t vector_store, std::conditional_t<GROUPED, gd_tile_group, gd_tile_rope> extra)
+                      uint32_t vector_store)
 {
-    auto &&rp = gd_tile_rope_of(extra);
     constexpr uint32_t BM = 64u * WM, BN = 64u * WN;
     constexpr int A_PER = BM / 32;                 /* 16-byte chunks of the activation tile per thread */
     constexpr int B_PER = W_NK ? (int)(BN / 32) : 8; /* weight chunks per thread */
@@ -152,10 +111,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
     unsigned char *epi = gd_tile_smem + STAGE_BYTES;           /* [64][BN] halfs */
     float *s_inv = reinterpret_cast<float *>(epi); /* [BM] row factors of rms_norm; live during the main loop only */
 
-    if constexpr (GROUPED) tiles_m = (uint32_t)__builtin_amdgcn_readfirstlane(extra.tiles[0]);
     const uint32_t total = tiles_m * tiles_n;
-    const gd_elem *wt = w;  /* GROUPED: the weights of the current tile's group */
-    uint32_t m_end = p.M;   /* GROUPED: one behind the last row of the group */
     constexpr bool DIRECT = PRO == GD_HIP_PRO_NONE;
     uint32_t m0 = 0u, n0 = 0u; /* origin of the current tile (rows, output columns) */
     /* swiglu epilogue ([N,K] weights of 2H rows, H = p.N output columns).  The BN weight rows of a tile are two
@@ -168,15 +124,6 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
     auto wrow = [&](uint32_t tn0, uint32_t r) __attribute__((always_inline)) {
         const uint32_t wc = r / (BN / 2u), wr = r % (BN / 2u);
         return gated ? (wr < HW ? tn0 + wc * HW + wr : p.swiglu_cols + tn0 + wc * HW + (wr - HW)) : tn0 + r;
-    };
-    /* first of 8 weight rows that a direct load of tile rows r .. r + 7 fetches.  GROUPED: a last column tile of fewer
-     * outputs (N % 8 == 0) takes the direct path too, with its last rows again in place of those behind them; what they
-     * give is not stored */
-    auto wrow_direct = [&](uint32_t tn0, uint32_t r) __attribute__((always_inline)) -> uint32_t {
-        if constexpr (!GROUPED) return wrow(tn0, r);
-        const uint32_t wc = r / (BN / 2u), wr = r % (BN / 2u);
-        if (!gated) return min(tn0 + r, p.N - 8u);
-        return (wr < HW ? 0u : p.swiglu_cols) + min(tn0 + wc * HW + wr % HW, p.N - 8u);
     };
     auto wrow_ok = [&](uint32_t tn0, uint32_t r) __attribute__((always_inline)) {
         return (gated ? tn0 + (r / (BN / 2u)) * HW + r % HW : tn0 + r) < p.N;
@@ -191,37 +138,21 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         const uint32_t gsz = min(tiles_m - first_m, 8u);
         const uint32_t row_tile = first_m + (pid % width) % gsz;
         tn0 = ((pid % width) / gsz) * out_bn;
-        if constexpr (GROUPED) {
-            const uint32_t group = (uint32_t)__builtin_amdgcn_readfirstlane(extra.tiles[2u + 2u * row_tile]);
-            tm0 = (uint32_t)__builtin_amdgcn_readfirstlane(extra.tiles[3u + 2u * row_tile]);
-            wt = w + (size_t)group * extra.w_rows * p.ldw;
-            m_end = (uint32_t)__builtin_amdgcn_readfirstlane(extra.first[group + 1u]);
-        } else {
-            tm0 = row_tile * BM;
-        }
+        tm0 = row_tile * BM;
     };
     auto direct_ok = [&](uint32_t tm0, uint32_t tn0) __attribute__((always_inline)) {
-        return DIRECT && (GROUPED || (tm0 + BM <= p.M && tn0 + out_bn <= p.N)) && (p.K % 64u) == 0u && p.K >= 128u;
+        return DIRECT && tm0 + BM <= p.M && tn0 + out_bn <= p.N && (p.K % 64u) == 0u && p.K >= 128u;
     };
 
     uint32_t tid_opaque = threadIdx.x;
     bool prefetched = false; /* the first two K tiles of the current output tile are already requested */
-#ifdef GD_TILE_TIMELINE
-    uint32_t timeline_tile = 0xffffffffu;
-#endif
     for (uint32_t tile = blockIdx.x; tile < total; tile += gridDim.x) {
-#ifdef GD_TILE_TIMELINE
-    ++timeline_tile;
-    const unsigned long long timeline_c0 = __builtin_amdgcn_s_memtime();
-    GD_TILE_NOTE(0, __builtin_amdgcn_s_memrealtime());
-#endif
     /* Everything below is derived from the thread id anew for every tile: were it loop-invariant, the
      * compiler would hoist some hundred addresses and offsets out of the tile loop and spill them. */
     asm volatile("" : "+v"(tid_opaque));
     const uint32_t tid = tid_opaque, lane = tid & 63u, wave = tid >> 6;
     const uint32_t wm = wave >> 1, wn = wave & 1u;
     locate(tile, m0, n0);
-    const uint32_t row_end = GROUPED ? m_end : p.M; /* for the epilogue: m_end moves on with the next tile's loads */
 
     /* staging coordinates */
     const uint32_t a_c = tid & 7u, a_r = tid >> 3; /* activation: chunk a_c of rows a_r + 32*i */
@@ -247,7 +178,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 ra[i] = zero8;
                 if (PRO == GD_HIP_PRO_SWIGLU) rz[i] = zero8;
             }
-            if (!GUARDED || (kok && gm < m_end)) {
+            if (!GUARDED || (kok && gm < p.M)) {
                 const gd_elem *xr = x + (size_t)gm * p.ldx + k;
                 ra[i] = *reinterpret_cast<const gd_elem8 *>(xr);
                 if (PRO == GD_HIP_PRO_SWIGLU) rz[i] = *reinterpret_cast<const gd_elem8 *>(xr + p.K);
@@ -260,7 +191,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 const uint32_t gn = wrow(n0, a_r + 32u * (uint32_t)i);
                 if (GUARDED) rb[i] = zero8;
                 if (!GUARDED || (kok && wrow_ok(n0, a_r + 32u * (uint32_t)i)))
-                    rb[i] = *reinterpret_cast<const gd_elem8 *>(wt + (size_t)gn * p.ldw + k);
+                    rb[i] = *reinterpret_cast<const gd_elem8 *>(w + (size_t)gn * p.ldw + k);
             }
         } else {
             const uint32_t gn = n0 + kb_nc * 8u;
@@ -269,7 +200,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 const uint32_t gk = kt * GD_TILE_BK + kb_j * 8u + i;
                 if (GUARDED || !KB_ALL) rb[i] = zero8;
                 if ((KB_ALL || kb_active) && (!GUARDED || (gk < p.K && gn < p.N)))
-                    rb[i] = *reinterpret_cast<const gd_elem8 *>(wt + (size_t)gk * p.ldw + gn);
+                    rb[i] = *reinterpret_cast<const gd_elem8 *>(w + (size_t)gk * p.ldw + gn);
             }
         }
     };
@@ -342,7 +273,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         } else if (W_NK) {
             const uint32_t tb = t - (uint32_t)A_DIRECT;
             const uint32_t row0 = wave_u * (BN / 4u) + tb * RW;
-            gd_tile_load_lds16(wt + (size_t)wrow_direct(tn0, row0) * p.ldw + kt * DBK, (tb & 1u) ? d_off_b1 : d_off_b,
+            gd_tile_load_lds16(w + (size_t)wrow(tn0, row0) * p.ldw + kt * DBK, (tb & 1u) ? d_off_b1 : d_off_b,
                                lds_base + ((2u * BM + stage * BN) * CH + row0 * CH) * 16u);
         } else {
             /* k-rows kr0 .. kr0+RPL-1 of the tile; lane L fills position L%CPR of row kr0 + L/CPR */
@@ -350,7 +281,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
             const uint32_t kr0 = (wave_u * (uint32_t)B_DIRECT + tb) * RPL;
             const uint32_t row = (RPL >= 4u ? 0u : ((tb * RPL) & 3u)) + lane / CPR; /* row & 3 */
             const uint32_t chunk = (lane % CPR) ^ ((row & 3u) << 2);
-            gd_tile_load_lds16(wt + (size_t)(kt * DBK + kr0) * p.ldw + tn0, d_off_b + chunk * 16u,
+            gd_tile_load_lds16(w + (size_t)(kt * DBK + kr0) * p.ldw + tn0, d_off_b + chunk * 16u,
                                lds_base + ((2u * BM + stage * BN) * CH + kr0 * CPR) * 16u);
         }
     };
@@ -600,7 +531,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
                 const uint32_t idx = idx0 + tid;
                 const uint32_t er = idx / (CPRW / 2u), v = idx % (CPRW / 2u);
                 const uint32_t gr = m0 + (er >> 5) * (WM * 32u) + (uint32_t)I * 32u + (er & 31u), gc = n0 + v * 8u;
-                if (gr >= row_end || gc >= p.N) continue;
+                if (gr >= p.M || gc >= p.N) continue;
                 /* staged columns: wavefront column wc holds its HW value columns, then their gates */
                 const uint32_t cv = (v / (HW / 8u)) * (HW / 4u) + v % (HW / 8u);
                 gd_elem8 h = read_chunk(er, cv);
@@ -622,7 +553,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
             const uint32_t idx = idx0 + tid;
             const uint32_t er = idx / CPRW, v = idx % CPRW;
             const uint32_t gr = m0 + (er >> 5) * (WM * 32u) + (uint32_t)I * 32u + (er & 31u), gc = n0 + v * 8u;
-            if (gr >= row_end || gc >= p.N) continue;
+            if (gr >= p.M || gc >= p.N) continue;
             gd_elem8 h = read_chunk(er, v);
             gd_elem *yr = y + (size_t)gr * p.ldy + gc;
             if (vector_store && gc + 8u <= p.N) {
@@ -783,130 +714,8 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         if (WM > 3) pass(std::integral_constant<int, (WM > 3 ? 3 : 0)>{});
     };
 
-    /* ROPE instantiation (whole tiles only; the launcher sees to that): the wavefront's 128 columns lie inside q, k
-     * or v (hd is a multiple of 256) and hold whole heads, so both columns of a rotation pair (c, c + half_d) are in
-     * one lane's accumulators: tiles j and j + half_d / 32.  Rounding points as in the separate operators: the
-     * projection is rounded to F16 (with its bias), rotated in F32 with the angles of the row's position, rounded
-     * again.  Rotated quads then take the path of epilogue_own; a row piece goes to row m of q or to row
-     * cache_row[m] of the K or V cache. */
-    auto epilogue_own_rope = [&](auto mode_tag) __attribute__((always_inline)) {
-        if (decltype(mode_tag)::value != GD_HIP_EPI_NONE) load_bias();
-        unsigned char *own = epi + wave * 8192u;
-        const uint32_t rr = lane >> 4, v = lane & 15u;
-        const uint32_t col0 = n0 + wn * (WN * 32u);
-        const uint32_t region = col0 >= 2u * rp.hd ? 2u : (col0 >= rp.hd ? 1u : 0u); /* q, k, v */
-        gd_elem *dst = rp.q;
-        if (region == 1u) dst = rp.k_cache;
-        if (region == 2u) dst = rp.v_cache;
-        dst += col0 - region * rp.hd + v * 8u;
-        const uint32_t row_w = m0 + wm * (WM * 32u);
-        typedef float gd_float4v __attribute__((ext_vector_type(4)));
-        /* What a pass needs from memory: the angles of its 32 rows (region q or k) and the destination rows of the
-         * lane's 8 row pieces.  Both are requested one pass ahead so that their latency passes behind the pass in
-         * front: the angles into the registers the running pass has just used them from, the rows into a second
-         * set.
-         * table_at: element offset of the lane's first angle of pass I in the angle tables, which are laid out for this read
-         * (blocks of 32 rows, groups of 8 pairs, the low and the high 4 pairs of all 32 rows: the 64 lanes of a load
-         * read 1 KB of consecutive memory; group g of the block lies 256 elements behind group g - 1); a signed
-         * 32-bit number (the launcher keeps the tables below 2^31 elements), so that the loads take the table's base
-         * from scalar registers and the constant steps as immediate offsets */
-        auto table_at = [&](int I) __attribute__((always_inline)) {
-            return (int32_t)(((row_w >> 5) + (uint32_t)I) * (rp.half_d * 32u) + frag_c * 128u + frag_row * 4u);
-        };
-        auto request_rows = [&](int I, int32_t (&drow)[8]) __attribute__((always_inline)) {
-#pragma unroll
-            for (uint32_t it = 0; it < 8u; ++it) {
-                const uint32_t r = row_w + (uint32_t)I * 32u + it * 4u + rr;
-                drow[it] = region == 0u ? (int32_t)r : rp.cache_row[r];
-            }
-        };
-        auto pass = [&](auto pass_tag, auto t_tag, gd_float4v (&cs)[8], gd_float4v (&sn)[8], const int32_t (&drow)[8],
-                        int32_t (&drow_next)[8]) __attribute__((always_inline)) {
-            constexpr int I = decltype(pass_tag)::value;
-            constexpr int T = decltype(t_tag)::value; /* accumulator tiles per half head */
-            constexpr bool MORE = I + 1 < WM;
-            if (MORE) request_rows(I + 1, drow_next);
-            auto stage = [&](int j, int pr, gd_elem4 a, gd_elem4 b) __attribute__((always_inline)) {
-                const uint32_t c = (uint32_t)j * 4u + 2u * (uint32_t)pr + frag_c;
-                *reinterpret_cast<gd_elem8 *>(own + (frag_row * 16u + (c ^ (frag_row & 15u))) * 16u) = pair_chunk(a, b);
-            };
-            if (region < 2u) {
-                const int32_t tnext = table_at(I + 1);
-#pragma unroll
-                for (int t = 0; t < T; ++t) {
-#pragma unroll
-                    for (int pr = 0; pr < 2; ++pr) {
-                        gd_elem4 olo[WN / (2 * T)][2], ohi[WN / (2 * T)][2];
-#pragma unroll
-                        for (int s2 = 0; s2 < 2; ++s2) {
-                            const int q = 2 * pr + s2;
-#pragma unroll
-                            for (int g = 0; g < WN / (2 * T); ++g) {
-                                const int jlo = g * 2 * T + t, jhi = jlo + T;
-                                const gd_elem4 lo = quad_f16(mode_tag, acc[I][jlo], jlo, q);
-                                const gd_elem4 hi = quad_f16(mode_tag, acc[I][jhi], jhi, q);
-#pragma unroll
-                                for (int r = 0; r < 4; ++r) {
-                                    gd_elem a, b;
-                                    gd_rope_rotate((float)lo[r], (float)hi[r], cs[t * 4 + q][r], sn[t * 4 + q][r], &a, &b);
-                                    olo[g][s2][r] = a;
-                                    ohi[g][s2][r] = b;
-                                }
-                            }
-                            if (MORE) {
-                                cs[t * 4 + q] = *reinterpret_cast<const gd_float4v *>(rp.cos + (tnext + 256 * (t * 4 + q)));
-                                sn[t * 4 + q] = *reinterpret_cast<const gd_float4v *>(rp.sin + (tnext + 256 * (t * 4 + q)));
-                            }
-                        }
-#pragma unroll
-                        for (int g = 0; g < WN / (2 * T); ++g) {
-                            stage(g * 2 * T + t, pr, olo[g][0], olo[g][1]);
-                            stage(g * 2 * T + t + T, pr, ohi[g][0], ohi[g][1]);
-                        }
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-#pragma unroll
-                    for (int pr = 0; pr < 2; ++pr)
-                        stage(j, pr, quad_f16(mode_tag, acc[I][j], j, 2 * pr), quad_f16(mode_tag, acc[I][j], j, 2 * pr + 1));
-            }
-            gd_elem8 h[8];
-#pragma unroll
-            for (uint32_t it = 0; it < 8u; ++it) {
-                const uint32_t e = it * 4u + rr;
-                h[it] = *reinterpret_cast<const gd_elem8 *>(own + (e * 16u + (v ^ (e & 15u))) * 16u);
-            }
-#pragma unroll
-            for (uint32_t it = 0; it < 8u; ++it) {
-                if (drow[it] >= 0) *reinterpret_cast<gd_elem8 *>(dst + (size_t)(uint32_t)drow[it] * rp.hd) = h[it];
-            }
-        };
-        auto passes = [&](auto t_tag) __attribute__((always_inline)) {
-            constexpr int T = decltype(t_tag)::value;
-            gd_float4v cs[8], sn[8];
-            int32_t even[8], odd[8];
-            request_rows(0, even);
-            if (region < 2u) {
-                const int32_t t0 = table_at(0);
-#pragma unroll
-                for (int t = 0; t < T * 4; ++t) {
-                    cs[t] = *reinterpret_cast<const gd_float4v *>(rp.cos + (t0 + 256 * t));
-                    sn[t] = *reinterpret_cast<const gd_float4v *>(rp.sin + (t0 + 256 * t));
-                }
-            }
-            pass(std::integral_constant<int, 0>{}, t_tag, cs, sn, even, odd);
-            pass(std::integral_constant<int, 1>{}, t_tag, cs, sn, odd, even);
-            pass(std::integral_constant<int, (WM > 2 ? 2 : 0)>{}, t_tag, cs, sn, even, odd);
-            pass(std::integral_constant<int, (WM > 2 ? 3 : 0)>{}, t_tag, cs, sn, odd, even);
-        };
-        if (rp.half_d == 64u) passes(std::integral_constant<int, (WN >= 4 ? 2 : 1)>{});
-        else passes(std::integral_constant<int, 1>{});
-    };
-
         /* interior tile: every staged chunk is in range, so the main loop carries no guards */
-        const bool interior = m0 + BM <= m_end && n0 + out_bn <= p.N && (p.K % GD_TILE_BK) == 0u;
+        const bool interior = m0 + BM <= p.M && n0 + out_bn <= p.N && (p.K % GD_TILE_BK) == 0u;
 
         if (PRO == GD_HIP_PRO_RMS_NORM) {
             __syncthreads(); /* the previous tile's epilogue has left the buffer that holds the row factors */
@@ -958,7 +767,7 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
             const uint32_t next = tile + gridDim.x;
             if (next < total) {
                 uint32_t nm0, nn0;
-                locate(next, nm0, nn0); /* GROUPED: also the group of the next tile, whose loads are requested here */
+                locate(next, nm0, nn0);
                 if (direct_ok(nm0, nn0)) {
                     direct_loads(nm0, nn0, 0u);
                     direct_loads(nm0, nn0, 1u);
@@ -979,14 +788,8 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
             }
         }
 
-#ifdef GD_TILE_TIMELINE
-        GD_TILE_NOTE(1, __builtin_amdgcn_s_memrealtime());
-        GD_TILE_NOTE(3, __builtin_amdgcn_s_memtime() - timeline_c0);
-#endif
         auto finish = [&](auto mode_tag) __attribute__((always_inline)) {
-            if constexpr (ROPE) {
-                epilogue_own_rope(mode_tag);
-            } else if (WM >= 3 && WN == 4 && vector_store && m0 + BM <= row_end && n0 + out_bn <= p.N) {
+            if (WM == 4 && WN == 4 && vector_store && m0 + BM <= p.M && n0 + out_bn <= p.N) {
                 if (gated) epilogue_own_gated(mode_tag);
                 else epilogue_own(mode_tag);
             } else {
@@ -996,65 +799,9 @@ gd_linear_tile_kernel(const gd_elem *__restrict__ x, const gd_elem *__restrict__
         if (p.epilogue == GD_HIP_EPI_BIAS_F32) finish(std::integral_constant<uint32_t, GD_HIP_EPI_BIAS_F32>{});
         else if (p.epilogue == GD_HIP_EPI_BIAS_F16) finish(std::integral_constant<uint32_t, GD_HIP_EPI_BIAS_F16>{});
         else finish(std::integral_constant<uint32_t, GD_HIP_EPI_NONE>{});
-        GD_TILE_NOTE(2, __builtin_amdgcn_s_memrealtime());
     }
 }
 
-/* Streaming stores for outputs larger than the L2s together: what reads a smaller one finds part of it there.  Two projections, a
- * gated one and a normalised residual addition behind them, BF16, us, with ordinary and with streaming stores: 2048 rows of 2048
- * columns (outputs of 17, 23 and 8 MB) 232.5 (247.5), 4096 x 1024 (17, 23, 8) 137.4 (145.1); 16384 x 1024 (67, 92, 34) 470 (457),
- * 16384 x 2048 (134, 185, 67) 1421 (1400).  Where the line lies between, whole prefills with all stores streaming, and streaming
- * beyond 32 and from 64 MiB on: 18,000 rows of a 512-column F16 decoder (outputs of 19 to 57 MB) 2109, 2107, 2122; 12,500 rows
- * 878, 879, 887; the BF16 layers of 2048 columns, 3,500 rows (14 to 60 MB) 3828, 3825, 3810; 13,600 rows of 1024 columns
- * 6734, 6737, 6713; others differ by less.  A reader of a larger output pays: the norms and rotations of 24,000 latent rows 31 ->
- * 36 us. */
-#define GD_TILE_STREAM_BYTES (32u << 20)
-static inline gd_hip_linear_params gd_tile_streamed(const gd_hip_linear_params &params)
-{
-    gd_hip_linear_params p = params;
-    if ((uint64_t)p.M * p.N * 2u > GD_TILE_STREAM_BYTES) p.flags |= GD_HIP_LINEAR_STREAM_Y;
-    return p;
-}
-
-#ifdef GD_LINEAR_TILE_GROUPED
-template <int WM, int WN>
-static int launch_tile_grouped(hipStream_t stream, const gd_elem *x, const gd_elem *w, gd_elem *y,
-                               const gd_hip_linear_params &p, const gd_tile_group &group, uint32_t max_tiles,
-                               uint32_t workgroups)
-{
-    constexpr uint32_t BM = 64u * WM, BN = 64u * WN;
-    constexpr size_t lds = (size_t)2u * (BM + BN) * 8u * 16u + (size_t)64u * BN * 2u;
-    static bool configured = false;
-    auto kernel = gd_linear_tile_kernel<WM, WN, true, GD_HIP_PRO_NONE, false, true>;
-    if (!configured) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return (int)e;
-        configured = true;
-    }
-    const uint32_t out_bn = p.swiglu_cols != 0u ? BN / 2u : BN, tiles_n = (p.N + out_bn - 1u) / out_bn;
-    const uint64_t all = (uint64_t)max_tiles * tiles_n;
-    kernel<<<(uint32_t)(all < workgroups ? all : workgroups), 256, lds, stream>>>(x, w, nullptr, nullptr, nullptr, y, p,
-                                                                                  max_tiles, tiles_n, 1u, group);
-    return (int)hipGetLastError();
-}
-
-/* y rows packed by group = x rows times the group's weights: p as for gd_hip_launch_linear_tile (M: packed rows; [N,K]
- * weights, N % 8 == 0, 16-byte aligned rows of x, w and y, no bias, no residual); max_tiles: upper bound of the row tiles, of 256
- * (big_tiles) or 128 rows */
-extern "C" int gd_hip_launch_linear_tile_grouped_bf16(hipStream_t stream, const void *x, const void *w, void *y,
-                                                      const gd_hip_linear_params *p, const int32_t *first,
-                                                      const int32_t *tiles, uint32_t w_rows, uint32_t max_tiles,
-                                                      int big_tiles, int compute_units)
-{
-    const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
-    const gd_tile_group group = {first, tiles, w_rows};
-    const gd_hip_linear_params s = gd_tile_streamed(*p);
-    if (big_tiles)
-        return launch_tile_grouped<4, 4>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, s, group, max_tiles, units);
-    return launch_tile_grouped<2, 2>(stream, (const gd_elem *)x, (const gd_elem *)w, (gd_elem *)y, s, group, max_tiles, 2u * units);
-}
-#else
 template <int WM, int WN, bool W_NK, int PRO>
 int gd_linear_tile_launch_one(hipStream_t stream, const gd_elem *x, const gd_elem *w, const gd_elem *bias,
                            const gd_elem *residual, const gd_elem *norm_w, gd_elem *y, const gd_hip_linear_params &p,
@@ -1074,8 +821,7 @@ int gd_linear_tile_launch_one(hipStream_t stream, const gd_elem *x, const gd_ele
     const uint32_t tiles_m = (p.M + BM - 1u) / BM, tiles_n = (p.N + out_bn - 1u) / out_bn;
     /* persistent workgroups: at most `workgroups` of them (a multiple of 8 keeps the tile -> XCD relation) */
     const uint32_t grid = tiles_m * tiles_n < workgroups ? tiles_m * tiles_n : workgroups;
-    kernel<<<grid, 256, lds, stream>>>(x, w, bias, residual, norm_w, y, p, tiles_m, tiles_n, vector_store,
-                                       gd_tile_rope{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0u, 0u});
+    kernel<<<grid, 256, lds, stream>>>(x, w, bias, residual, norm_w, y, p, tiles_m, tiles_n, vector_store);
     return (int)hipGetLastError();
 }
 
@@ -1096,14 +842,12 @@ GD_TILE_PROLOGUES(, 4, 4, false)
 #elif defined(GD_LINEAR_TILE_PART) && GD_LINEAR_TILE_PART == 3
 GD_TILE_PROLOGUES(, 2, 2, true)
 GD_TILE_PROLOGUES(, 2, 2, false)
-GD_TILE_FORM(, 3, 4, true, GD_HIP_PRO_NONE)
 #else
 #if !GD_LINEAR_IS_BF16
 GD_TILE_PROLOGUES(extern, 4, 4, true)
 GD_TILE_PROLOGUES(extern, 4, 4, false)
 GD_TILE_PROLOGUES(extern, 2, 2, true)
 GD_TILE_PROLOGUES(extern, 2, 2, false)
-GD_TILE_FORM(extern, 3, 4, true, GD_HIP_PRO_NONE)
 #endif
 
 template <int WM, int WN>
@@ -1127,6 +871,11 @@ static int launch_tile(hipStream_t stream, const gd_elem *x, const gd_elem *w, c
 #undef GD_GO
 }
 
+/* linear_tile_nk.hip: [N,K] weights without a prologue */
+extern "C" int GD_LINEAR_FN(gd_hip_try_launch_linear_tile_nk)(hipStream_t stream, const void *x, const void *w, const void *bias,
+                                                const void *residual, void *y, const gd_hip_linear_params *params,
+                                                int vector_store, uint32_t units);
+
 /* Requires: K % 8 == 0, 16-byte aligned x rows (and gate half), w rows (for [K,N]: N % 8 == 0 too) and
  * norm weight; M >= 1.  big_tiles: use the 256 x 256 tile (one workgroup per compute unit; the 128 x 128 tile
  * fits two). */
@@ -1139,6 +888,8 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear_tile)(hipStream_t stream, const
     const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
     const gd_elem *xp = (const gd_elem *)x, *rp = (const gd_elem *)residual;
     gd_elem *yp = (gd_elem *)y;
+    const int e = GD_LINEAR_FN(gd_hip_try_launch_linear_tile_nk)(stream, x, w, bias, residual, y, &p, vector_store, units);
+    if (e >= 0) return e;
     if (big_tiles) {
         /* The persistent workgroups walk whole rounds of 256 x 256 tiles; a last round that fills only part of the
          * compute units costs a full tile time.  When that costs more than it would with small tiles, the rows of
@@ -1155,37 +906,18 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear_tile)(hipStream_t stream, const
             const double whole = (double)((tiles + units - 1u) / units);
             const double cut = (double)(((uint64_t)head_m * tiles_n + units - 1u) / units) +
                                0.35 * (double)((small + 2u * units - 1u) / (2u * units));
-            /* a tail that small tiles would need more than one round for, and that fits one round of 192 x 256
-             * tiles (three row tiles per wavefront instead of four): one launch of those; measured on the
-             * 2048-column projections of the scaled decoder (5,653 tail rows: 720 small tiles on 512 places, or 248
-             * tiles of 192 rows, or 240 when the launch is anchored at the last row, see below) */
-            const uint32_t mid_rows = (tail_rows + 191u) / 192u * 192u;
-            const uint64_t mid = (uint64_t)(mid_rows / 192u) * tiles_n;
-            /* whole tiles only (a ragged row tile would leave the direct staging path and take twice as long as the
-             * others of its round): the launch covers the LAST mid_rows rows, so its first rows, fewer than 192,
-             * are rows of the head launch computed once more, to the same bits (the same products in the same
-             * order, the same epilogue); that needs an output the residual does not alias */
+            /* whole row tiles when the output allows it (a ragged row tile would leave the direct staging path and take
+             * twice as long as the others of its round): the launch covers the LAST rows, so its first rows, fewer than
+             * 128, are rows of the head launch computed once more, to the same bits; that needs an output the residual
+             * does not alias */
             const bool apart = rp == nullptr || rp + (size_t)p.M * p.ldr <= yp || yp + (size_t)p.M * p.ldy <= rp;
-            const bool mid_tiles = p.w_is_nk && p.prologue == GD_HIP_PRO_NONE && p.swiglu_cols == 0u &&
-                                   small > 2u * units && mid <= units && mid_rows <= p.M && (p.N % 256u) == 0u &&
-                                   vector_store && apart;
-            if (mid_tiles || cut + 0.1 < whole) {
+            if (cut + 0.1 < whole) {
                 gd_hip_linear_params head = p, tail = p;
-                int e;
                 head.M = head_rows;
                 tail.M = tail_rows;
-                e = launch_tile<4, 4>(stream, xp, (const gd_elem *)w, (const gd_elem *)bias, rp, (const gd_elem *)norm_w,
-                                      yp, head, (uint32_t)vector_store, units);
-                if (e != (int)hipSuccess) return e;
-                if (mid_tiles) {
-                    const uint32_t first = p.M - mid_rows;
-                    tail.M = mid_rows;
-                    return gd_linear_tile_launch_one<3, 4, true, GD_HIP_PRO_NONE>(
-                        stream, xp + (size_t)first * p.ldx, (const gd_elem *)w, (const gd_elem *)bias,
-                        rp != nullptr ? rp + (size_t)first * p.ldr : nullptr, (const gd_elem *)norm_w,
-                        yp + (size_t)first * p.ldy, tail, (uint32_t)vector_store, units);
-                }
-                /* small tiles: whole row tiles as well when the output allows it (anchored at the last row) */
+                const int e4 = launch_tile<4, 4>(stream, xp, (const gd_elem *)w, (const gd_elem *)bias, rp, (const gd_elem *)norm_w,
+                                                 yp, head, (uint32_t)vector_store, units);
+                if (e4 != (int)hipSuccess) return e4;
                 uint32_t first = head_rows;
                 const uint32_t up = (tail_rows + 127u) / 128u * 128u;
                 if (apart && up <= p.M) {
@@ -1204,54 +936,4 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear_tile)(hipStream_t stream, const
                              (uint32_t)vector_store, 2u * units);
 }
 
-#if !GD_LINEAR_IS_BF16
-/* The qkv projection of a packed prefill with rotation and cache append in the epilogue (gd_tile_rope): x [M,K],
- * w [3*hd, K], whole 256 x 256 tiles only.  Requires: M % 256 == 0, hd % 256 == 0, K % 64 == 0, K >= 128, 16-byte
- * aligned rows of x, w, q and the caches, half_d 32 or 64 (head size 64 or 128). */
-extern "C" int GD_LINEAR_FN(gd_hip_launch_linear_tile_rope)(hipStream_t stream, const void *x, const void *w, const void *bias,
-                                              const gd_hip_linear_params *params, const float *cos_rows,
-                                              const float *sin_rows, const int32_t *cache_row, void *q, void *k_cache,
-                                              void *v_cache, uint32_t hd, uint32_t half_d, int compute_units)
-{
-    const gd_hip_linear_params &p = *params;
-    constexpr size_t lds = (size_t)2u * (256u + 256u) * 8u * 16u + (size_t)64u * 256u * 2u;
-    static bool configured = false;
-    auto kernel = gd_linear_tile_kernel<4, 4, true, GD_HIP_PRO_NONE, true>;
-    if (p.M == 0u) return (int)hipSuccess;
-    if ((p.M % 256u) != 0u || (hd % 256u) != 0u || p.N != 3u * hd || (p.K % 64u) != 0u || p.K < 128u || !p.w_is_nk ||
-        p.prologue != GD_HIP_PRO_NONE || p.has_residual || p.swiglu_cols != 0u || (half_d != 32u && half_d != 64u))
-        return (int)hipErrorInvalidValue;
-    if (!configured) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        if (e != hipSuccess) return (int)e;
-        configured = true;
-    }
-    const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
-    const uint32_t tiles_m = p.M / 256u, tiles_n = p.N / 256u;
-    const uint32_t grid = tiles_m * tiles_n < units ? tiles_m * tiles_n : units;
-    kernel<<<grid, 256, lds, stream>>>((const gd_elem *)x, (const gd_elem *)w, (const gd_elem *)bias, nullptr, nullptr,
-                                       nullptr, p, tiles_m, tiles_n, 1u,
-                                       gd_tile_rope{cos_rows, sin_rows, cache_row, (gd_elem *)q, (gd_elem *)k_cache,
-                                                    (gd_elem *)v_cache, hd, half_d});
-    return (int)hipGetLastError();
-}
-
-/* Row tiles of 256 that fill whole rounds of `units` workgroups for an [M, N] output in 256-column tiles: the rows
- * the rope form takes; the rest (a partly filled last round, a ragged last row tile) goes through the plain
- * projection and the table-driven rotation kernel. */
-extern "C" uint32_t GD_LINEAR_FN(gd_hip_linear_tile_rope_head_rows)(uint32_t M, uint32_t N, int compute_units)
-{
-    const uint32_t units = ((uint32_t)(compute_units > 0 ? compute_units : 256) + 7u) & ~7u;
-    const uint32_t tiles_n = (N + 255u) / 256u, whole_m = M / 256u;
-    const uint64_t tiles = (uint64_t)whole_m * tiles_n;
-    const uint64_t rounds = tiles / units;
-    uint32_t head_m = rounds != 0u ? (uint32_t)(rounds * units / tiles_n) : 0u;
-    /* a few tiles beyond whole rounds cost less than they would in small tiles only when the remainder is nearly a
-     * round itself */
-    if (tiles - (uint64_t)head_m * tiles_n >= (uint64_t)units * 3u / 4u) head_m = whole_m;
-    return head_m * 256u;
-}
-#endif
 #endif /* GD_LINEAR_TILE_PART */
-#endif /* GD_LINEAR_TILE_GROUPED */

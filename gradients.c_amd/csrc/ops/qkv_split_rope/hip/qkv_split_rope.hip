@@ -194,7 +194,7 @@ __host__ __device__ __forceinline__ uint64_t gd_rope_table_at(uint64_t n, uint32
 }
 
 /* Angles and cache rows of the N packed prompt rows, computed once per prefill and used by every layer's qkv
- * projection (the rotation epilogue of the tile kernel in ops/linear/hip/linear_tile.hip and the row kernel below):
+ * projection (the rotation epilogue of the tile kernel in ops/linear/hip/linear_tile_nk.hip and the row kernel below):
  * cos_rows / sin_rows F32 (laid out by gd_rope_table_at) with the same arithmetic as the rotation kernels above, cache_row [N] = sequence *
  * tmax + seq_pos[sequence] + token under the rules of the packed append (nothing unless cu starts at 0; a sequence with
  * a negative position or whose rows do not fit behind it is skipped), -1 for a row that is not appended. */

@@ -31,6 +31,8 @@ static uint32_t tile_rows_of(const gd_backend_routed_args *a, uint32_t rows, uin
 {
     const uint64_t per_expert = (uint64_t)rows * a->top / a->experts;
     if (dtype != GD_BACKEND_DTYPE_BF16 || (a->width % 8u) != 0u || (a->ff % 8u) != 0u) return GD_ROUTED_ANY_ROWS;
+    /* byte offsets within an expert's weights are 31-bit numbers in the tile kernel */
+    if (4ull * a->ff * a->width > 0x7fffffffu || a->ff > 0x3fffffu || a->width > 0x3fffffu) return GD_ROUTED_ANY_ROWS;
     if (per_expert >= 768u) return GD_ROUTED_WIDE_ROWS;
     return per_expert >= 24u ? GD_ROUTED_TILE_ROWS : GD_ROUTED_STREAM_ROWS;
 }

@@ -1037,12 +1037,57 @@ def test_many_row_projection_prologues(backend, arena, oracle, M, K, N, nk):
     _close(y.read(), oracle.linear(oracle.rms_norm(x, nw, 1e-5), w_kn, bias))
 
 
+# [N,K] weights without a prologue: tiles of 256, 192 and 128 rows, two K tiles of which the second is empty (K = 8, 56), K and
+# N that end inside a chunk row, rows behind the last whole tile; the last three: 192-row tiles, 256-row tiles, two whole rounds of
+# 256-row tiles with the other rows in 128-row ones
+@pytest.mark.parametrize("M,K,N", [(128, 8, 8), (129, 56, 264), (255, 72, 40), (300, 136, 1000), (2050, 200, 8200), (9500, 1000, 2048),
+                                   (13000, 1000, 2040), (20001, 1496, 2048)])
+def test_many_row_projection_of_nk_weights_edges(backend, arena, oracle, gda, M, K, N):
+    """Every bias mode, residual and gate, into rows of a wider matrix: nothing is written beside them.  Bound: the sum's own
+    rounding (an F16 unit of the projection before the bias, of the bias sum, of the residual sum)."""
+    x = oracle.normal_f16((M, K), 2600 + K, 1.0)
+    w = oracle.normal_f16((2 * N, K), 2601 + N, 0.1)
+    bias = oracle.normal_f16((2 * N,), 2602, 0.5)
+    res = oracle.normal_f16((M, N), 2603, 1.0)
+    tx, tr = arena.from_numpy(x), arena.from_numpy(res)
+    wide = arena.alloc((M + 1, N + 16), 1)
+
+    class Part:
+        def matrix(self):
+            return gda.MatrixView(wide.buffer.handle, wide.offset, M, N, (N + 16) * 2, gda.F16)
+
+    u = x.astype(np.float32) @ w.astype(np.float32).T
+    b32, r32 = bias.astype(np.float32), res.astype(np.float32)
+
+    def check(want, size, weights, biased, **form):
+        wide.write(np.full((M + 1, N + 16), 77.0, np.float16))
+        backend.fused_linear(tx, weights, biased, form.get("residual"), None, Part(), True, form.get("mode", 0), 0,
+                             epilogue=form.get("epilogue", 0))
+        got = wide.read()
+        assert np.all(got[M:] == 77.0) and np.all(got[:, N:] == 77.0)
+        err = np.abs(got[:M, :N].astype(np.float32) - want)
+        assert np.all(err <= 1e-3 * size + 1e-4), (form, float((err - 1e-3 * size).max()))
+
+    wn, bn, first = arena.from_numpy(w[:N].copy()), arena.from_numpy(bias[:N].copy()), u[:, :N]
+    sum_, size = first + b32[:N], np.abs(first) + np.abs(b32[:N])
+    check(first, np.abs(first), wn, None)
+    check(sum_, size, wn, bn, mode=2)
+    check(sum_, np.abs(sum_), wn, bn, mode=1)
+    check(first + r32, np.abs(first) + np.abs(first + r32), wn, None, residual=tr)
+    check(sum_ + r32, size + np.abs(sum_) + np.abs(sum_ + r32), wn, bn, mode=2, residual=tr)
+    # value and gate are rounded before the product, whose factors grow by at most 1.1 of a change of the gate
+    value, gate = u[:, :N] + b32[:N], u[:, N:] + b32[N:]
+    silu = gate / (1 + np.exp(-gate))
+    size = (np.abs(u[:, :N]) + np.abs(b32[:N]) + np.abs(value)) * np.abs(silu)
+    size += 1.1 * np.abs(value) * (np.abs(u[:, N:]) + np.abs(b32[N:]) + np.abs(gate)) + np.abs(value * silu)
+    check(value * silu, size, arena.from_numpy(w), arena.from_numpy(bias), mode=2, epilogue=1)
+
+
 @pytest.mark.parametrize("K", [128, 192])
 def test_many_row_projection_tail_in_192_row_tiles(backend, arena, oracle, K):
-    """13,192 rows onto 2048 columns of an [N,K] weight: 52 x 8 tiles of 256 x 256 are 1.6 rounds on 256 compute units;
-    the first round's 8,192 rows run in those tiles, the 5,000 rows behind them (640 tiles of 128 x 128 would need more
-    than one round of them) in one launch of 27 x 8 tiles of 192 x 256, three row tiles per wavefront, the last row tile
-    ragged.  Whole output against the oracle, plain, with bias, and with bias and residual."""
+    """13,192 rows onto 2048 columns of an [N,K] weight: more than whole rounds of any tile on 256 compute units, the last
+    row tile ragged.  Whole output against the oracle, plain, with bias, and with bias and residual; and the same bits for
+    the first rows of a call that other tiles may take."""
     M, N = 13192, 2048
     x = oracle.normal_f16((M, K), 2500 + K, 1.0)
     w = oracle.normal_f16((N, K), 2501, 0.05)
@@ -1056,8 +1101,7 @@ def test_many_row_projection_tail_in_192_row_tiles(backend, arena, oracle, K):
     inter = oracle.linear_nt(x, w, bias)
     got = y.read()
     _close(got, oracle.add(res, inter), through=inter)
-    # the 192-row launch starts at row 13192 - 27 * 192 = 8008: rows 8008..8191 are rows of the first launch computed
-    # once more.  The same rows from a call over the first 8,192 rows alone (whole 256 x 256 tiles only): same bits
+    # the first 8,192 rows from a call of their own: the same products in the same order whatever the tile
     y_head = arena.alloc((8192, N), 1)
     backend.fused_linear(tx.rows(0, 8192), tw, tb, tr.rows(0, 8192), None, y_head, True, 2, 0)
     assert np.array_equal(_bits(y_head.read()), _bits(got[:8192]))
@@ -1067,8 +1111,7 @@ def test_many_row_projection_full_size_sampled(backend, oracle):
     """The packed-prefill projections of BASELINE config 4 at full size (30,229 rows): the qkv projection ([N,K]
     weight, bias added after the F16 rounding) and the down projection ([K,N] weight, F32 bias, residual), operands
     filled on the device, sampled rows (first, last, both sides of every kind of tile edge) against float64; and the
-    attention projection with its residual on an [N,K] weight, whose 5,653 rows behind the last whole round of 256 x 256
-    tiles go to one launch of 192 x 256 tiles (rows 24,576 on; tile edges every 192 rows, the last tile ragged)."""
+    attention projection with its residual on an [N,K] weight (a last, partly filled round of tiles, the last one ragged)."""
     M = 30229
     big = backend.buffer(900 << 20)
     try:
