@@ -9,8 +9,10 @@
  * weight fragment is the first operand: lane l holds row l % 16 of a tile and its columns 4 (l / 16) .. + 3.
  *
  * Staging.  K tiles of 64 through two LDS stages, filled by buffer loads that write LDS (8 rows of 128 bytes per
- * instruction); chunk c (16 bytes) of row r sits at c ^ (r & 7) ^ (r >> 3 & 1), so that the 16 rows a fragment read
- * touches lie in different banks.  Rows behind the operand's end are out of the descriptor's range: they cost no
+ * instruction); chunk c (16 bytes) of row r sits at c ^ (r >> 1 & 7).  A 16-byte read is served in groups of 16 lanes,
+ * 0 to 3, 12 to 15 and 20 to 27 the first of them: rows 0 to 3 and 12 to 15 of one chunk and rows 4 to 11 of the next,
+ * which this puts into all 64 banks (with c ^ (r & 7) ^ (r >> 3 & 1), right for fragments of 32 rows, half of the
+ * cycles in which the LDS was busy were conflicts).  Rows behind the operand's end are out of the descriptor's range: they cost no
  * traffic, and nothing they give is stored.  Columns behind K get such addresses too, and with them zeros.  So ragged
  * tiles run like whole ones.
  *
@@ -178,16 +180,16 @@ gd_linear_tile_nk_kernel(const gd_elem *__restrict__ x, const gd_elem *__restric
      * gated tile holds, per wavefront column, BN/4 value rows and then the gate rows of the same outputs, so that a lane
      * has value and gate of an output in its own accumulators (tiles j and j + TN/2). */
     const uint32_t pitch_x = p.ldx * 2u, pitch_w = p.ldw * 2u; /* bytes */
-    const uint32_t chunk = (lane & 7u) ^ ((lane >> 3) & 7u);
+    const uint32_t chunk = (lane & 7u) ^ (lane >> 4); /* of rows 16 n .. + 7; of the 8 rows behind them chunk ^ 4 */
     const uint32_t row_x = wave * (BM / 4u);
     const uint32_t row_w = KIND == GD_NK_GATED ? (wave & 1u) * p.swiglu_cols + (wave >> 1) * (BN / 4u) : wave * (BN / 4u);
     /* byte offsets of the lane's chunk in every load: in vector registers, because a scalar offset is not part of the
      * range check */
     uint32_t at_x[TM], at_w[TN];
 #pragma unroll
-    for (uint32_t t = 0; t < (uint32_t)TM; ++t) at_x[t] = (row_x + 8u * t + (lane >> 3)) * pitch_x + (chunk ^ (t & 1u)) * 16u;
+    for (uint32_t t = 0; t < (uint32_t)TM; ++t) at_x[t] = (row_x + 8u * t + (lane >> 3)) * pitch_x + (chunk ^ (t & 1u) * 4u) * 16u;
 #pragma unroll
-    for (uint32_t t = 0; t < (uint32_t)TN; ++t) at_w[t] = (row_w + 8u * t + (lane >> 3)) * pitch_w + (chunk ^ (t & 1u)) * 16u;
+    for (uint32_t t = 0; t < (uint32_t)TN; ++t) at_w[t] = (row_w + 8u * t + (lane >> 3)) * pitch_w + (chunk ^ (t & 1u) * 4u) * 16u;
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     uint32_t lds_x = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + row_x * 128u));
     uint32_t lds_w = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds0 + B_AT + wave * (BN / 4u) * 128u));
@@ -220,7 +222,7 @@ gd_linear_tile_nk_kernel(const gd_elem *__restrict__ x, const gd_elem *__restric
     /* ---- fragments: lane l reads chunk l / 16 (+ 4 in the second half of K) of row l % 16 */
     gd_elem8 fa[2][TM], fb[2][TN];
     gd_nk_float4 acc[TM][TN];
-    const uint32_t frag = (lane & 15u) * 128u + (((lane >> 4) ^ (lane & 7u) ^ ((lane >> 3) & 1u)) << 4);
+    const uint32_t frag = (lane & 15u) * 128u + (((lane >> 4) ^ ((lane >> 1) & 7u)) << 4);
     /* [0]: first half of the next K tile, [1]: second half of this */
     uint32_t from_a[2] = {wm * (TM * 2048u) + frag, wm * (TM * 2048u) + (frag ^ 64u)};
     uint32_t from_b[2] = {B_AT + wn * (TN * 2048u) + frag, B_AT + wn * (TN * 2048u) + (frag ^ 64u)};
@@ -452,7 +454,7 @@ gd_linear_tile_nk_kernel(const gd_elem *__restrict__ x, const gd_elem *__restric
     auto cut = [&]() __attribute__((always_inline)) {
         const int32_t left = (int32_t)p.K - (int32_t)(kr * 64u);
         if (left >= 64) return;
-        const uint32_t even = (int32_t)(chunk * 8u) < left ? 0u : 0x80000000u, odd = (int32_t)((chunk ^ 1u) * 8u) < left ? 0u : 0x80000000u;
+        const uint32_t even = (int32_t)(chunk * 8u) < left ? 0u : 0x80000000u, odd = (int32_t)((chunk ^ 4u) * 8u) < left ? 0u : 0x80000000u;
 #pragma unroll
         for (int t = 0; t < TM; ++t) at_x[t] ^= (t & 1) ? odd : even;
 #pragma unroll
