@@ -22,12 +22,20 @@
  * the multiply-add in front of the exp2, and the running maximum of a row moves (O and the row sum rescaled) only
  * when a block raises it by more than 8 binary orders: the result does not depend on the reference point.
  *
+ * What it takes (32 prompts of 64 to 2048 rows, 16 heads of 128): 355 us, 410 before the key rows' addresses, the clearing of V
+ * rows and the zeroing of score registers left the loop (buffer descriptors that follow the block and end with the segment;
+ * fragment addresses computed once; the first product over a zero accumulator), before masks became plain comparisons with the
+ * row's limits (branches per key before: 16 prompts of 20 to 400 rows through a window of 256, 8 heads of 64, 33.7 -> 15.1 us),
+ * and before the longest prompts came first.  Vector and matrix instructions are each busy a third of the time; wavefronts wait
+ * at the block's barrier and for each other.
+ *
  * LDS layouts (16-byte chunks, CPR = D/8 per row).  K: chunk c of key row r at position c ^ (r & 15)
  * (D = 128) or c ^ ((r >> 1) & 7) (D = 64): the 16 lanes of a fragment read hit 16 different bank groups.
  * V: chunk c of key row r at c ^ ((r & 3) << 2) (D = 128) or c ^ (((r >> 1) & 1) << 2) (D = 64): the four
  * key rows of a transposing read cover all banks.
  */
-#include "../../_shared/hip_device.h"
+#include "../../_shared/hip_row_blocks.h"
+#include <type_traits>
 
 #define GD_VL_NEG_INF (-__builtin_inff())
 
@@ -39,39 +47,19 @@ struct gd_hip_sdpa_varlen_params {
                          segment b in cache row t of sequence b */
 };
 
-__device__ __forceinline__ bool gd_vl_allowed(int i, int j, int causal, int window, int prefix_len)
-{
-    if (causal) {
-        if (prefix_len > 0) {
-            if (i < prefix_len) {
-                if (j >= prefix_len) return false;
-            } else if (j > i) {
-                return false;
-            }
-        } else if (j > i) {
-            return false;
-        }
-    }
-    if (window > 0) {
-        if (prefix_len > 0) {
-            if (i >= prefix_len && j >= prefix_len && (i - j) >= window) return false;
-        } else if ((i - j) >= window) {
-            return false;
-        }
-    }
-    return true;
-}
+typedef int gd_vl_int4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) unsigned char gd_vl_lds;
 
-/* 16 bytes per lane from global memory straight into LDS (lane l's data lands at lds_address + 16*l).
- * Assembly, because the compiler would otherwise wait for every outstanding load before each LDS read;
- * the kernel places its own s_waitcnt vmcnt. */
-__device__ __forceinline__ void gd_vl_load_lds16(const gd_half *uniform_base, uint32_t lane_byte_offset,
-                                                 uint32_t lds_byte_address)
+/* 16 bytes per lane from global memory straight into LDS (lane l's data lands at lds + IMM + 16 l); lanes behind the
+ * descriptor's range get zeros.  Assembly, because the compiler would otherwise wait for every outstanding load before
+ * each LDS read; the kernel places its own s_waitcnt vmcnt. */
+template <int IMM>
+__device__ __forceinline__ void gd_vl_load_lds16(gd_vl_int4 descriptor, uint32_t lane_bytes, uint32_t lds)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, 0 offen lds"
                  :
-                 : "s"(lds_byte_address), "v"(lane_byte_offset), "s"(uniform_base)
-                 : "memory");
+                 : "s"(lds), "n"(IMM), "v"(lane_bytes), "s"(descriptor)
+                 : "memory", "scc");
 }
 
 template <int D>
@@ -94,45 +82,16 @@ gd_sdpa_varlen_mfma_kernel(const gd_half *__restrict__ q, const gd_half *__restr
     const uint32_t hq = blockIdx.x % p.hq, pair = blockIdx.x / p.hq;
     const uint32_t hkv = hq / (p.hq / p.hkv);
 
-    /* (segment, 128-row block) number `pair`: lane t of the wavefront takes segment t of a run of 64 segments (one
-     * load of cu per lane instead of a chain of dependent scalar loads, which cost a workgroup of a short prompt as
-     * much as its attention), the blocks of the run are summed across the lanes, and the first lane whose running
-     * count passes `pair` names the segment */
     if (cu[0] < 0) return;
-    uint32_t seen = 0u, b = p.batch;
-    int start = 0, end = 0;
-    for (uint32_t b0 = 0u; b0 < p.batch; b0 += 64u) {
-        const uint32_t bl = b0 + lane;
-        int s0 = 0, e0 = 0;
-        if (bl < p.batch) {
-            s0 = cu[bl];
-            e0 = cu[bl + 1u];
-        }
-        const uint32_t nb = e0 > s0 ? ((uint32_t)(e0 - s0) + BQ - 1u) / BQ : 0u;
-        uint32_t incl = nb; /* inclusive sum over the lanes below and this one */
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const uint32_t up = (uint32_t)__shfl_up((int)incl, off, 64);
-            if ((int)lane >= off) incl += up;
-        }
-        const unsigned long long hit = __builtin_amdgcn_ballot_w64(seen + incl > pair);
-        if (hit != 0ull) {
-            const int src = __builtin_ctzll(hit);
-            b = b0 + (uint32_t)src;
-            start = __shfl(s0, src, 64);
-            end = __shfl(e0, src, 64);
-            seen += (uint32_t)__shfl((int)(incl - nb), src, 64);
-            break;
-        }
-        seen += (uint32_t)__shfl((int)incl, 63, 64);
-    }
-    if (b == p.batch || end > (int)p.n_rows) return;
+    gd_row_block at;
+    if (!gd_find_row_block(cu, p.batch, BQ, pair, &at) || at.end > (int)p.n_rows) return;
+    const uint32_t b = at.seq;
+    const int start = at.start, end = at.end;
     const int T_len = end - start;
     if (p.kv_tmax != 0u && (uint32_t)T_len > p.kv_tmax) return; /* a segment its cache cannot hold: out stays */
-    /* first and last row of K and V this workgroup may touch */
+    /* row of K and V that holds the segment's first key */
     const uint32_t kv_first = p.kv_tmax != 0u ? b * p.kv_tmax : (uint32_t)start;
-    const uint32_t kv_last = p.kv_tmax != 0u ? b * p.kv_tmax + (p.kv_tmax - 1u) : p.n_rows - 1u;
-    const int i0 = (int)((pair - seen) * BQ);
+    const int i0 = (int)(at.block * BQ);
     const int causal = (int)p.causal, window = (int)p.window, prefix = (int)p.prefix_len;
 
     /* key blocks this workgroup walks */
@@ -156,22 +115,43 @@ gd_sdpa_varlen_mfma_kernel(const gd_half *__restrict__ q, const gd_half *__restr
         if (row_live) qf[ks] = *reinterpret_cast<const gd_half8 *>(q + q_elem + 16 * ks + 8 * h);
     }
 
-    const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)gd_vl_smem;
-    const gd_half *k_head = k + (size_t)hkv * D, *v_head = v + (size_t)hkv * D;
+    /* Staging.  A load of this wavefront fills RPL key rows; lane offsets do not depend on the block, whose rows the
+     * descriptor's base and range follow: rows behind the segment's end (another segment's, or a cache's free ones) arrive
+     * as zeros, so that probability 0 times their values is 0. */
+    gd_vl_lds *const smem = (gd_vl_lds *)gd_vl_smem;
     const uint32_t row_pitch = p.hkv * D * 2u; /* bytes between consecutive key rows */
-    auto issue_block = [&](int jb, uint32_t stage) __attribute__((always_inline)) {
+    const uint32_t lds_wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(uintptr_t)smem + wave * (uint32_t)LOADS * 1024u));
+    uint32_t off_k[LOADS], off_v[LOADS];
 #pragma unroll
-        for (int t = 0; t < LOADS; ++t) {
-            const uint32_t r0 = (wave * (uint32_t)LOADS + (uint32_t)t) * RPL;
-            const uint32_t r = r0 + lane / CPR, pos = lane % CPR;
-            const uint32_t grow = min(kv_first + (uint32_t)jb + r, kv_last); /* stays inside the tensor */
-            const uint32_t ck = pos ^ (D == 128 ? (r & 15u) : ((r >> 1) & 7u));
-            const uint32_t cv = pos ^ (D == 128 ? ((r & 3u) << 2) : (((r >> 1) & 1u) << 2));
-            const uint32_t dst = lds_base + (stage * 2u * TILE_CHUNKS + r0 * CPR) * 16u;
-            gd_vl_load_lds16(k_head, grow * row_pitch + ck * 16u, dst);
-            gd_vl_load_lds16(v_head, grow * row_pitch + cv * 16u, dst + TILE_CHUNKS * 16u);
+    for (int t = 0; t < LOADS; ++t) {
+        const uint32_t r = (wave * (uint32_t)LOADS + (uint32_t)t) * RPL + lane / CPR, pos = lane % CPR;
+        off_k[t] = r * row_pitch + (pos ^ (D == 128 ? (r & 15u) : ((r >> 1) & 7u))) * 16u;
+        off_v[t] = r * row_pitch + (pos ^ (D == 128 ? ((r & 3u) << 2) : (((r >> 1) & 1u) << 2))) * 16u;
+    }
+    const uint32_t segment = (uint32_t)__builtin_amdgcn_readfirstlane((int)kv_first);
+    const uint32_t keys = (uint32_t)__builtin_amdgcn_readfirstlane(T_len);
+    /* the key block jb of K or V (part 0, 1) into a stage; jb < keys */
+    auto request = [&](auto part, int jb, uint32_t stage) __attribute__((always_inline)) {
+        constexpr int V = decltype(part)::value, AT = V * (int)TILE_CHUNKS * 16;
+        const uint64_t first = (uint64_t)(V ? v : k) + (uint64_t)(segment + (uint32_t)jb) * row_pitch + hkv * D * 2u;
+        const uint32_t range = min(keys - (uint32_t)jb - 1u, BKEYS - 1u) * row_pitch + D * 2u;
+        gd_vl_int4 of;
+        of[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)first);
+        of[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(first >> 32));
+        of[2] = __builtin_amdgcn_readfirstlane((int)range);
+        of[3] = 0x00020000; /* untyped, no swizzle */
+        const uint32_t to = lds_wave + stage * (2u * TILE_CHUNKS * 16u);
+        const uint32_t (&off)[LOADS] = V ? off_v : off_k;
+        gd_vl_load_lds16<AT>(of, off[0], to);
+        gd_vl_load_lds16<AT + 1024>(of, off[1], to);
+        if constexpr (LOADS == 4) {
+            gd_vl_load_lds16<AT + 2048>(of, off[LOADS - 2], to);
+            gd_vl_load_lds16<AT + 3072>(of, off[LOADS - 1], to);
         }
     };
+    using gd_k = std::integral_constant<int, 0>;
+    using gd_v = std::integral_constant<int, 1>;
+    static_assert(LOADS == 2 || LOADS == 4, "the loads above");
 
     gd_float16 o[DTILES];
 #pragma unroll
@@ -181,47 +161,58 @@ gd_sdpa_varlen_mfma_kernel(const gd_half *__restrict__ q, const gd_half *__restr
     float m = GD_VL_NEG_INF, l = 0.f;
     const float scale2 = p.scale * 1.4426950408889634f;
     const bool plain_causal = causal != 0 && window == 0 && prefix == 0;
-    const int jmax = min(i, T_len - 1); /* last visible key of this lane's row under plain causal attention */
+    /* visible keys of this lane's row: up to jmax, but for jfrom .. jgone */
+    int jmax = T_len - 1;
+    if (causal) jmax = min(jmax, prefix > 0 && i < prefix ? prefix - 1 : i);
+    const int jgone = window > 0 && (prefix == 0 || i >= prefix) ? i - window : -1, jfrom = prefix;
 
-    /* transposing read coordinates of this lane: group g = lane/16 -> channel block 16*(g&1), key half g/2 == h;
-     * lane q + 4e of a group addresses key row e, channels 4q .. 4q+3 */
+    /* Fragment addresses in the first stage; what a step of K or of the channels changes is a xor with a constant, key rows
+     * and the V block are immediate offsets.
+     * K: key row lq (+ 32 t), chunk 2 ks + h.  V, transposing reads: group g = lane / 16 -> channel block 16 (g & 1), key
+     * half g / 2 == h; lane q + 4 e of a group addresses key row e (+ 4 h + 16 ts, + 8 the second), channels 4 q .. + 3. */
     const uint32_t tr_q = lane & 3u, tr_e = (lane >> 2) & 3u, tr_g1 = (lane >> 4) & 1u;
+    const uint32_t v_row = 4u * h + tr_e; /* the swizzle of rows 8 and 16 ts behind it is the same */
+    uint32_t at_k[KSTEPS], at_v[DTILES];
+#pragma unroll
+    for (uint32_t ks = 0; ks < (uint32_t)KSTEPS; ++ks)
+        at_k[ks] = (lq * CPR + ((2u * ks + h) ^ (D == 128 ? (lq & 15u) : ((lq >> 1) & 7u)))) * 16u;
+#pragma unroll
+    for (uint32_t dt = 0; dt < (uint32_t)DTILES; ++dt)
+        at_v[dt] = (TILE_CHUNKS + v_row * CPR + ((4u * dt + 2u * tr_g1 + (tr_q >> 1)) ^ (D == 128 ? (tr_e << 2) : (((v_row >> 1) & 1u) << 2)))) * 16u +
+                   (tr_q & 1u) * 8u;
 
-    issue_block(kbeg, 0u);
-    uint32_t it = 0u;
-    for (int jb = kbeg; jb < kend; jb += (int)BKEYS, ++it) {
-        const uint32_t stage = it & 1u;
-        __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): this wavefront's share of block jb is in LDS */
-        __syncthreads();                    /* everyone's share is, and the other stage is no longer read */
-        if (jb + (int)BKEYS < kend) issue_block(jb + (int)BKEYS, stage ^ 1u);
-        const unsigned char *sK = gd_vl_smem + (size_t)stage * 2u * TILE_CHUNKS * 16u;
-        const unsigned char *sV = sK + TILE_CHUNKS * 16u;
-        if (jb + (int)BKEYS > T_len) {
-            /* last, partial block: rows past the segment hold another segment's values; their probabilities
-             * are zero, but 0 * inf would still poison the sum, so clear those V rows */
-            const uint32_t first = (uint32_t)(T_len - jb);
-            for (uint32_t c = first * CPR + tid; c < TILE_CHUNKS; c += 256u)
-                reinterpret_cast<gd_u128 *>(const_cast<unsigned char *>(sV))[c] = gd_u128{0u, 0u, 0u, 0u};
-            __syncthreads();
-        }
-        /* a causal wavefront whose rows all precede the block has nothing to add */
+    /* The scores of a block are computed while the block in front of it is exponentiated: matrix and vector instructions of
+     * one wavefront side by side.  So K runs a block ahead of V. */
+    auto key = [&](uint32_t stage, int n) __attribute__((always_inline)) { /* fragment n = t * KSTEPS + ks */
+        return *(__attribute__((address_space(3))) gd_half8 *)(smem + stage * (2u * TILE_CHUNKS * 16u) + at_k[n % KSTEPS] +
+                                                               32u * (uint32_t)(n / KSTEPS) * CPR * 16u);
+    };
+    auto value = [&](uint32_t stage, int n) __attribute__((always_inline)) {
+        gd_vl_lds *const at = smem + stage * (2u * TILE_CHUNKS * 16u) + at_v[n % DTILES] + 16u * (uint32_t)(n / DTILES) * CPR * 16u;
+        union { gd_short4 s[2]; gd_half8 hv; } u;
+        u.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gd_short4 *)at);
+        u.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gd_short4 *)(at + 8u * CPR * 16u));
+        return u.hv;
+    };
+    gd_float16 st0[2], st1[2];
+    request(gd_k{}, kbeg, 0u);
+    request(gd_v{}, kbeg, 0u);
+    if (kbeg + (int)BKEYS < kend) request(gd_k{}, kbeg + (int)BKEYS, 1u);
+    __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0) */
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < 2 * KSTEPS; ++n)
+        st0[n / KSTEPS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(key(0u, n), qf[n % KSTEPS], n % KSTEPS == 0 ? (gd_float16)(0.f) : st0[n / KSTEPS], 0, 0, 0);
+    /* block jb, whose K and V lie in `stage`: its scores st, the next block's go to `next` */
+    auto walk = [&](gd_float16 (&st)[2], gd_float16 (&next)[2], int jb, auto stage_tag) __attribute__((always_inline)) {
+        constexpr uint32_t stage = decltype(stage_tag)::value;
+        __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): this wavefront's share of V of block jb and of the next K is in LDS */
+        __syncthreads();                    /* everyone's share is; K of block jb and V of the one in front are no longer read */
+        if (jb + (int)BKEYS < kend) request(gd_v{}, jb + (int)BKEYS, stage ^ 1u);
+        if (jb + 2 * (int)BKEYS < kend) request(gd_k{}, jb + 2 * (int)BKEYS, stage);
+        /* a causal wavefront whose rows all precede the block has nothing to add, nor from the blocks behind it */
         const bool wave_needs = !causal || jb <= wi0 + 31 || (prefix > 0 && jb < prefix);
-        if (!wave_needs) continue;
-
-        /* S^T = K Q^T for the two 32-key tiles */
-        gd_float16 st[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) st[t][e] = 0.f;
-            const uint32_t r = 32u * t + lq;
-            const uint32_t swz = D == 128 ? (r & 15u) : ((r >> 1) & 7u);
-#pragma unroll
-            for (int ks = 0; ks < KSTEPS; ++ks) {
-                const gd_half8 kf = *reinterpret_cast<const gd_half8 *>(sK + (r * CPR + ((2u * ks + h) ^ swz)) * 16u);
-                st[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf, qf[ks], st[t], 0, 0, 0);
-            }
-        }
+        if (!wave_needs) return;
 
         /* scale, mask, block maximum.  The scores stay unscaled in their registers: scale2 > 0, so the maximum of the
          * raw values is the raw value of the maximum, and the scaling rides in the multiply-add in front of the exp2. */
@@ -229,15 +220,20 @@ gd_sdpa_varlen_mfma_kernel(const gd_half *__restrict__ q, const gd_half *__restr
                           (causal ? (prefix == 0 && jb + 63 <= wi0 && (window == 0 || wi0 + 31 - jb < window))
                                   : (window == 0));
         float mraw = GD_VL_NEG_INF;
-        if (!full) {
+        if (!full && plain_causal) { /* no window, no prefix: one comparison against min(i, T_len - 1) */
+            const int behind = jmax - jb - 4 * (int)h;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) st[t][e] = 32 * t + 8 * (e >> 2) + (e & 3) > behind ? GD_VL_NEG_INF : st[t][e];
+        } else if (!full) {
 #pragma unroll
             for (int t = 0; t < 2; ++t) {
 #pragma unroll
                 for (int e = 0; e < 16; ++e) {
                     const int j = jb + 32 * t + 8 * (e >> 2) + 4 * (int)h + (e & 3);
-                    /* plain causal attention (no window, no prefix): one comparison against min(i, T_len - 1) */
-                    if (plain_causal ? j > jmax : (j >= T_len || !gd_vl_allowed(i, j, causal, window, prefix)))
-                        st[t][e] = GD_VL_NEG_INF;
+                    const bool hidden = (j > jmax) | ((j <= jgone) & (j >= jfrom));
+                    st[t][e] = hidden ? GD_VL_NEG_INF : st[t][e];
                 }
             }
         }
@@ -264,38 +260,44 @@ gd_sdpa_varlen_mfma_kernel(const gd_half *__restrict__ q, const gd_half *__restr
                 for (int e = 0; e < 16; ++e) o[t][e] *= corr;
         }
         const float msafe = m == GD_VL_NEG_INF ? 0.f : m;
+        /* probabilities of this block beside the scores of the next (of stale keys behind the last block: not used) */
+        constexpr int NK = 2 * KSTEPS, PER = 32 / NK, AHEAD = 4;
         float psum = 0.f;
-        gd_half8 pf[4];
+        gd_half8 pf[4], kf[AHEAD], vf[AHEAD];
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int n = 0; n < AHEAD; ++n) kf[n] = key(stage ^ 1u, n);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
+        for (int n = 0; n < NK; ++n) {
+            next[n / KSTEPS] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[n % AHEAD], qf[n % KSTEPS], n % KSTEPS == 0 ? (gd_float16)(0.f) : next[n / KSTEPS], 0, 0, 0);
+            if (n + AHEAD < NK) kf[n % AHEAD] = key(stage ^ 1u, n + AHEAD);
+            else vf[n + AHEAD - NK] = value(stage, n + AHEAD - NK);
+#pragma unroll
+            for (int x = n * PER; x < (n + 1) * PER; ++x) {
+                const int t = x / 16, e = x % 16;
                 const float pe = __builtin_amdgcn_exp2f(fmaf(st[t][e], scale2, -msafe));
                 psum += pe;
                 pf[2 * t + (e >> 3)][e & 7] = (gd_half)pe;
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
         l += psum;
 
-        /* O^T += V^T P^T: four 16-key steps, DTILES channel tiles */
+        /* O^T += V^T P^T: fragment n = channel tile n % DTILES of 16-key step n / DTILES, four of them on their way */
+        constexpr int NV = 4 * DTILES;
 #pragma unroll
-        for (int ts = 0; ts < 4; ++ts) {
-#pragma unroll
-            for (int dt = 0; dt < DTILES; ++dt) {
-                const uint32_t chunk = 4u * dt + 2u * tr_g1 + (tr_q >> 1);
-                const uint32_t r_lo = 16u * ts + 4u * h + tr_e; /* second read: + 8; both have r & 3 == tr_e */
-                const uint32_t swz_lo = D == 128 ? (tr_e << 2) : (((r_lo >> 1) & 1u) << 2);
-                const uint32_t swz_hi = D == 128 ? (tr_e << 2) : ((((r_lo + 8u) >> 1) & 1u) << 2);
-                const gd_short4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gd_short4 *)(
-                    sV + (r_lo * CPR + (chunk ^ swz_lo)) * 16u + (tr_q & 1u) * 8u));
-                const gd_short4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) gd_short4 *)(
-                    sV + ((r_lo + 8u) * CPR + (chunk ^ swz_hi)) * 16u + (tr_q & 1u) * 8u));
-                union { gd_short4 s[2]; gd_half8 hv; } u;
-                u.s[0] = lo;
-                u.s[1] = hi;
-                o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(u.hv, pf[ts], o[dt], 0, 0, 0);
-            }
+        for (int n = 0; n < NV; ++n) {
+            o[n % DTILES] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[n % AHEAD], pf[n / DTILES], o[n % DTILES], 0, 0, 0);
+            if (n + AHEAD < NV) vf[n % AHEAD] = value(stage, n + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
         }
+    };
+    for (int jb = kbeg; jb < kend;) {
+        walk(st0, st1, jb, std::integral_constant<uint32_t, 0>{});
+        jb += (int)BKEYS;
+        if (jb >= kend) break;
+        walk(st1, st0, jb, std::integral_constant<uint32_t, 1>{});
+        jb += (int)BKEYS;
     }
 
     /* normalise, then through LDS so that rows leave with 16-byte stores */
