@@ -8,7 +8,7 @@ int gd_hip_launch_latent_prepare(hipStream_t stream, const void *proj, uint32_t 
 int gd_hip_launch_latent_query(hipStream_t stream, const void *qv, const void *w_ukt, const float *angles, void *ql,
                                const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32, uint32_t units);
 int gd_hip_launch_latent_attend(hipStream_t stream, const void *ql, const void *cache, float *o_lat,
-                                const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32);
+                                const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32, uint32_t units);
 int gd_hip_launch_latent_value(hipStream_t stream, const float *o_lat, const void *w_uv, const void *gate, uint32_t ldg,
                                void *out, uint32_t rows, const gd_hip_latent_params *m, int is_f32, uint32_t units);
 
@@ -232,7 +232,7 @@ gd_status gd_backend_latent_attend(gd_backend *backend, const gd_backend_tensor_
                                        dtype == GD_BACKEND_DTYPE_F32, (uint32_t)backend->compute_units);
         if (e == 0)
             e = gd_hip_launch_latent_attend(backend->stream, wp + w.ql, gd_hip_view_ptr(cache), (float *)(wp + w.sums), &m,
-                                            &q, dtype == GD_BACKEND_DTYPE_F32);
+                                            &q, dtype == GD_BACKEND_DTYPE_F32, (uint32_t)backend->compute_units);
         if (e == 0)
             e = gd_hip_launch_latent_value(backend->stream, (float *)(wp + w.sums), gd_hip_view_ptr(&w_uv),
                                            gd_hip_matrix_ptr(gate), ldg, gd_hip_view_ptr(out), (uint32_t)rows, &m,

@@ -182,61 +182,129 @@ gd_latent_query_kernel(const T *__restrict__ qv, const T *__restrict__ w_ukt, co
     }
 }
 
-/* grid (rows, heads); o_lat F32 [rows, heads, kv_rank] */
-template <typename T>
-__global__ void __launch_bounds__(256)
-gd_latent_attend_kernel(const T *__restrict__ ql, const T *__restrict__ cache, float *__restrict__ o_lat,
-                        gd_hip_latent_params m, gd_hip_seqs q)
+/* Rows row0 .. row0 + R - 1 of one head, which see the first keys, keys + 1, .. rows of a cache slot: a thread per key for the scores,
+ * a thread per latent channel for the sums, blocks of 256 keys.  A row's operations and their order do not depend on R; a row that
+ * does not see a key of the others leaves it out. */
+template <typename T, int R>
+__device__ __forceinline__ void gd_latent_attend_rows(const T *__restrict__ ql, const T *__restrict__ rows, float *__restrict__ o_lat,
+                                                      const gd_hip_latent_params &m, uint32_t row0, uint32_t h, uint32_t keys,
+                                                      float *smem, float (*sp)[256], float (*red)[4])
 {
-    extern __shared__ float smem[]; /* query [pitch], sums [kv_rank] */
-    __shared__ float sp[256], red[4];
-    float *sq = smem, *so = smem + m.pitch;
-    const uint32_t row = blockIdx.x, h = blockIdx.y;
-    int32_t s, pos, slot;
-    if (!gd_seq_of_row(q, row, &s, &pos, &slot)) return;
-    const uint32_t keys = min((uint32_t)pos + 1u, m.tmax), used = m.kv_rank + m.rot_dim;
-    const T *src = ql + ((size_t)row * m.heads + h) * m.pitch, *rows = cache + (size_t)slot * m.tmax * m.pitch;
-    for (uint32_t c = threadIdx.x; c < used; c += 256u) sq[c] = (float)src[c];
-    for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) so[c] = 0.f;
-    float mx = -INFINITY, total = 0.f;
-    for (uint32_t k0 = 0; k0 < keys; k0 += 256u) {
+    const uint32_t used = m.kv_rank + m.rot_dim, wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+    float *sq = smem, *so = smem + R * used; /* queries [R][used], sums [R][kv_rank] */
+    uint32_t sees[R];
+    float mx[R], total[R], keep[R];
+    __syncthreads(); /* rows in front of these are done with the memory */
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        const T *src = ql + ((size_t)(row0 + r) * m.heads + h) * m.pitch;
+        for (uint32_t c = threadIdx.x; c < used; c += 256u) sq[r * used + c] = (float)src[c];
+        for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) so[r * m.kv_rank + c] = 0.f;
+        sees[r] = min(keys + r, m.tmax);
+        mx[r] = -INFINITY;
+        total[r] = 0.f;
+    }
+    for (uint32_t k0 = 0; k0 < sees[R - 1]; k0 += 256u) {
         __syncthreads();
         const uint32_t k = k0 + threadIdx.x;
-        float score = -INFINITY;
-        if (k < keys) {
-            float a[1];
-            gd_latent_row_dot<1>(sq, rows + (size_t)k * m.pitch, used, a);
-            score = a[0] * m.scale;
+        float score[R], p[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) score[r] = -INFINITY;
+        if (k < sees[R - 1]) {
+            float a[R];
+            gd_latent_row_dot<R>(sq, rows + (size_t)k * m.pitch, used, a);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (k < sees[r]) score[r] = a[r] * m.scale;
         }
         /* maximum of the block's scores */
-        float t = gd_wave_max(score);
-        if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = t;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float t = gd_wave_max(score[r]);
+            if (lane == 0u) red[r][wave] = t;
+        }
         __syncthreads();
-        t = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-        const float nmx = fmaxf(mx, t), keep = expf(mx - nmx);
-        const float p = k < keys ? expf(score - nmx) : 0.f;
-        sp[threadIdx.x] = p;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float t = fmaxf(fmaxf(red[r][0], red[r][1]), fmaxf(red[r][2], red[r][3]));
+            const float nmx = fmaxf(mx[r], t);
+            keep[r] = expf(mx[r] - nmx);
+            p[r] = k < sees[r] ? expf(score[r] - nmx) : 0.f;
+            sp[r][threadIdx.x] = p[r];
+            mx[r] = nmx;
+        }
+        __syncthreads(); /* the maxima are read */
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float t = gd_wave_sum(p[r]);
+            if (lane == 0u) red[r][wave] = t;
+        }
         __syncthreads();
-        total = total * keep + gd_block_sum<4>(p, red);
-        mx = nmx;
-        const uint32_t nk = min(keys - k0, 256u);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float t = 0.f;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) t += red[r][w];
+            total[r] = total[r] * keep[r] + t;
+        }
+        const uint32_t all = sees[0] > k0 ? min(sees[0] - k0, 256u) : 0u, any = min(sees[R - 1] - k0, 256u); /* keys that every, some row sees */
         for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u) {
-            float a = so[c] * keep;
+            float a[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[r] = so[(uint32_t)r * m.kv_rank + c] * keep[r];
             const T *kr = rows + (size_t)k0 * m.pitch + c;
             uint32_t j = 0;
-            for (; j + 16u <= nk; j += 16u) { /* sixteen rows requested together */
+            for (; j + 16u <= all; j += 16u) { /* sixteen rows requested together */
                 float v[16];
 #pragma unroll
                 for (uint32_t e = 0; e < 16u; ++e) v[e] = (float)kr[(size_t)(j + e) * m.pitch];
 #pragma unroll
-                for (uint32_t e = 0; e < 16u; ++e) a = fmaf(sp[j + e], v[e], a);
+                for (uint32_t e = 0; e < 16u; ++e)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) a[r] = fmaf(sp[r][j + e], v[e], a[r]);
             }
-            for (; j < nk; ++j) a = fmaf(sp[j], (float)kr[(size_t)j * m.pitch], a);
-            so[c] = a;
+            for (; j < any; ++j) {
+                const float v = (float)kr[(size_t)j * m.pitch];
+#pragma unroll
+                for (int r = 0; r < R; ++r) a[r] = k0 + j < sees[r] ? fmaf(sp[r][j], v, a[r]) : a[r];
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) so[(uint32_t)r * m.kv_rank + c] = a[r];
         }
     }
-    for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u)
-        o_lat[((size_t)row * m.heads + h) * m.kv_rank + c] = so[c] / total;
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r)
+        for (uint32_t c = threadIdx.x; c < m.kv_rank; c += 256u)
+            o_lat[((size_t)(row0 + r) * m.heads + h) * m.kv_rank + c] = so[r * m.kv_rank + c] / total[r];
+}
+
+/* grid (ceil(rows / R), heads); o_lat F32 [rows, heads, kv_rank].  R rows behind each other share a reading of their sequence's cache */
+template <typename T, int R>
+__global__ void __launch_bounds__(256)
+gd_latent_attend_kernel(const T *__restrict__ ql, const T *__restrict__ cache, float *__restrict__ o_lat,
+                        gd_hip_latent_params m, gd_hip_seqs q)
+{
+    extern __shared__ float smem[];
+    __shared__ float sp[R][256], red[R][4];
+    const uint32_t row0 = blockIdx.x * R, h = blockIdx.y, n = min(q.rows - row0, (uint32_t)R);
+    int32_t s[R], pos[R], slot[R];
+    bool there[R], together = n == (uint32_t)R;
+#pragma unroll
+    for (uint32_t r = 0; r < R; ++r) {
+        there[r] = r < n && gd_seq_of_row(q, row0 + r, &s[r], &pos[r], &slot[r]);
+        together = together && there[r] && s[r] == s[0];
+    }
+    if (together) {
+        gd_latent_attend_rows<T, R>(ql, cache + (size_t)slot[0] * m.tmax * m.pitch, o_lat, m, row0, h, (uint32_t)pos[0] + 1u, smem, sp, red);
+        return;
+    }
+    if constexpr (R > 1) { /* rows of different sequences */
+        for (uint32_t r = 0; r < n; ++r) {
+            int32_t one, at, place;
+            if (!gd_seq_of_row(q, row0 + r, &one, &at, &place)) continue;
+            gd_latent_attend_rows<T, 1>(ql, cache + (size_t)place * m.tmax * m.pitch, o_lat, m, row0 + r, h, (uint32_t)at + 1u, smem, sp, red);
+        }
+    }
 }
 
 /* grid (ceil(rows / R), heads); out [rows, heads * vdim].  R rows share a reading of the weights; a wavefront takes every fourth
@@ -327,15 +395,21 @@ extern "C" int gd_hip_launch_latent_query(hipStream_t stream, const void *qv, co
     return (int)hipGetLastError();
 }
 
+/* Rows that share a reading of the cache: as above, and where sequences have many rows (a group that lies in two sequences goes row by
+ * row), and LDS enough for four rows.  Six portions of 160 to 570 rows, 8 heads of 256 + 64 channels, mean of the
+ * three that share: 103 -> 80 us */
 extern "C" int gd_hip_launch_latent_attend(hipStream_t stream, const void *ql, const void *cache, float *o_lat,
-                                           const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32)
+                                           const gd_hip_latent_params *m, const gd_hip_seqs *q, int is_f32, uint32_t units)
 {
-    const dim3 grid(q->rows, m->heads);
     const size_t lds = (m->pitch + m->kv_rank) * sizeof(float);
     if (q->rows == 0u) return (int)hipSuccess;
     if (lds > 48u * 1024u) return (int)hipErrorInvalidValue;
-#define GD_GO(T) gd_latent_attend_kernel<T><<<grid, 256, lds, stream>>>((const T *)ql, (const T *)cache, o_lat, *m, *q)
-    if (is_f32) GD_GO(float); else GD_GO(gd_bf16);
+#define GD_GO(T, R) gd_latent_attend_kernel<T, R><<<dim3((q->rows + R - 1u) / R, m->heads), 256, R * lds, stream>>>((const T *)ql, (const T *)cache, o_lat, *m, *q)
+    if (gd_latent_rows_share(q->rows, m->heads, units) && q->rows / 16u >= q->seqs && 4u * lds <= 48u * 1024u) {
+        if (is_f32) GD_GO(float, 4); else GD_GO(gd_bf16, 4);
+    } else {
+        if (is_f32) GD_GO(float, 1); else GD_GO(gd_bf16, 1);
+    }
 #undef GD_GO
     return (int)hipGetLastError();
 }

@@ -532,6 +532,29 @@ def test_latent_attention_of_prompts_portions_and_steps(backend, gda, arena, L, 
     _near(got, want, dtype, factor=1.5 if dtype == BF16 else 10)
 
 
+@pytest.mark.parametrize("sizes", [(16, 24, 8, 16, 48), (33, 20, 6, 10, 21), (12, 32, 16, 24, 300)], ids=lambda s: "x".join(map(str, s)))
+def test_rows_that_share_a_reading_of_the_latents(backend, gda, arena, L, sizes):
+    """Three sequences of unequal length, portions that begin and end anywhere, so that groups of four rows lie on both sides of
+    256 keys and in two sequences: the plain result, and the bits that the same rows get in calls too small to share."""
+    runs = [(1, 250, 61), (0, 0, 119), (2, 503, 10)]
+    together, alone = (Latent(gda, backend, arena, L, F32, *sizes, tmax=520) for _ in range(2))
+    held = together.rng.standard_normal(together.cache.shape)
+    N, H, D, R, V, KV = sum(n for _, _, n in runs), *sizes
+    proj = together.rng.standard_normal((N, 24 + KV + R + H * V))
+    q = together.rng.standard_normal((N, H, D + R))
+    for la in (together, alone):
+        la.cache.write_float(held)
+    got, want = together.run(runs, q=q, proj=proj)
+    _near(got, want, F32, factor=10)
+    first = 0
+    for slot, start, n in runs:
+        for at in range(0, n, 7):
+            rows = slice(first + at, first + min(at + 7, n))
+            few, _ = alone.run([(slot, start + at, rows.stop - rows.start)], q=q[rows], proj=proj[rows])
+            assert np.array_equal(few, got[rows]), (slot, at)
+        first += n
+
+
 @pytest.mark.parametrize("tmax", [1024, 1025], ids=["8 pieces", "9 pieces"])
 @pytest.mark.parametrize("sizes", [(3, 72, 24, 56, 112), (17, 32, 16, 40, 64), (2, 136, 136, 96, 640)], ids=lambda s: "x".join(map(str, s)))
 def test_steps_whose_keys_are_cut_into_pieces(backend, gda, arena, L, sizes, tmax):
