@@ -70,4 +70,19 @@ __device__ __forceinline__ bool gd_find_row_block(const int32_t *__restrict__ cu
     return false;
 }
 
+/* Sequence number `n` by length, the longest first (of up to 64; of more, n itself), for workgroups that each take a whole sequence:
+ * lane t holds sequence t and counts those in front of it. */
+__device__ __forceinline__ uint32_t gd_sequence_by_length(const int32_t *__restrict__ cu, uint32_t batch, uint32_t n)
+{
+    if (batch > 64u || n >= batch) return n;
+    const uint32_t lane = threadIdx.x & 63u;
+    const int rows = lane < batch ? cu[lane + 1u] - cu[lane] : 0;
+    uint32_t rank = 0u;
+    for (uint32_t t = 0u; t < batch; ++t) {
+        const int other = __builtin_amdgcn_readlane(rows, (int)t);
+        rank += other > rows || (other == rows && t < lane) ? 1u : 0u;
+    }
+    return (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(lane < batch && rank == n));
+}
+
 #endif

@@ -1,6 +1,6 @@
 /*
- * Softmax weights of the BF16 attention kernels: two BF16 numbers each, the weight rounded and what the rounding left (16 bits
- * together), two weights at a time so that each conversion instruction makes two of them.
+ * F32 operands of BF16 matrix instructions (softmax weights, states, decays): two BF16 numbers each, the value rounded and what the
+ * rounding left (16 bits together), two values at a time so that each conversion instruction makes two of them.
  */
 #ifndef GD_OPS_SHARED_HIP_WEIGHT_PAIRS_H
 #define GD_OPS_SHARED_HIP_WEIGHT_PAIRS_H
@@ -8,7 +8,9 @@
 
 typedef float gd_float2v __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ void gd_weight_pair(float a, float b, gd_bf16x8 &rounded, gd_bf16x8 &rest, int at)
+/* elements at, at + 1 of two vectors */
+template <typename V>
+__device__ __forceinline__ void gd_weight_pair(float a, float b, V &rounded, V &rest, int at)
 {
     union { gd_bf16x2 h; uint32_t u; } r, s;
     r.h = __builtin_convertvector((gd_float2v){a, b}, gd_bf16x2);

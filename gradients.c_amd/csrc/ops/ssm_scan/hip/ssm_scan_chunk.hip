@@ -20,18 +20,13 @@
  *   S = B'^T X       32 x 32 tiles of the [NP, PT] state dealt out to the wavefronts
  * Tokens behind a sequence's end enter with dt = 0 and zero rows: they neither decay nor add.
  */
-#include "../../_shared/hip_device.h"
+#include "../../_shared/hip_row_blocks.h"
+#include "../../_shared/hip_weight_pairs.h"
 #include "hip_ssm_scan_types.h"
 
 #define GD_SC_L 64u
 #define GD_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0)
 typedef short gd_sc_short4 __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ void gd_sc_split(float v, gd_bf16 *hi, gd_bf16 *lo)
-{
-    *hi = (gd_bf16)v;
-    *lo = (gd_bf16)(v - (float)*hi);
-}
 
 /* 8 consecutive k (rows k0 .. k0+7 of an LDS tile [k][column], `stride` bytes per row) of column col0 + l % 32, for the
  * lane's half k0 = ... + 8 * (l / 32): two transposing reads of four rows each */
@@ -75,7 +70,9 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
     const uint32_t p0 = blockIdx.x * L::PT, h = blockIdx.y, N = m.state, P = m.vdim, inner = m.heads * P;
     const uint32_t g = h / (m.heads / m.groups), cols = min(P - p0, L::PT);
     int32_t first, n, start, slot;
-    if (!gd_seq_span(q, blockIdx.z, &first, &n, &start, &slot)) return;
+    /* the longest sequences first: a launch lasts as long as its last workgroup. With pair conversions and
+     * double-buffered fragments, medians of six launches: 16 prompts of 64 to 2048, 351 -> 304 us; 64 shorter ones, 120 -> 110 */
+    if (!gd_seq_span(q, gd_sequence_by_length(q.cu, q.seqs, blockIdx.z), &first, &n, &start, &slot)) return;
     float *st = states + ((size_t)slot * m.heads + h) * N * P + p0;
     const float rate = expf(a_log[h]) * 1.4426950408889634f, bias = dt_bias[h], skip = d_skip[h];
 
@@ -152,12 +149,7 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
             for (int a = 0; a < 4; ++a) {
                 gd_bf16x4 vh, vl;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    gd_bf16 hi, lo;
-                    gd_sc_split(S[t][4 * a + r], &hi, &lo);
-                    vh[r] = hi;
-                    vl[r] = lo;
-                }
+                for (int r = 0; r < 4; r += 2) gd_weight_pair(S[t][4 * a + r], S[t][4 * a + r + 1], vh, vl, r);
                 const uint32_t at = (32u * pb + lc) * L::BC + (32u * nb + 8u * (uint32_t)a + 4u * hh) * 2u;
                 *reinterpret_cast<gd_bf16x4 *>(sm + L::sh + at) = vh;
                 *reinterpret_cast<gd_bf16x4 *>(sm + L::sl + at) = vl;
@@ -172,18 +164,26 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
         gd_float16 gm, ys;
 #pragma unroll
         for (int e = 0; e < 16; ++e) gm[e] = ys[e] = 0.f;
+        {
+            /* the fragments of a step are requested while the one in front of it is multiplied, here and in the other products */
+            gd_bf16x8 cv[2], ah[2], al[2], bv[2];
+            auto fetch = [&](int ks) __attribute__((always_inline)) {
+                const uint32_t c = (16u * (uint32_t)ks + 8u * hh) * 2u;
+                cv[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::c + i * L::BC + c);
+                bv[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::b + (32u * jb + lc) * L::BC + c);
+                ah[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::sh + (32u * pb + lc) * L::BC + c);
+                al[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::sl + (32u * pb + lc) * L::BC + c);
+            };
+            fetch(0);
 #pragma unroll
-        for (int ks = 0; ks < NP / 16; ++ks) {
-            const uint32_t c = (16u * ks + 8u * hh) * 2u;
-            const gd_bf16x8 cv = *reinterpret_cast<const gd_bf16x8 *>(sm + L::c + i * L::BC + c);
-            const gd_bf16x8 ah = *reinterpret_cast<const gd_bf16x8 *>(sm + L::sh + (32u * pb + lc) * L::BC + c);
-            const gd_bf16x8 al = *reinterpret_cast<const gd_bf16x8 *>(sm + L::sl + (32u * pb + lc) * L::BC + c);
-            if (jb <= ib) {
-                const gd_bf16x8 bv = *reinterpret_cast<const gd_bf16x8 *>(sm + L::b + (32u * jb + lc) * L::BC + c);
-                gm = GD_MFMA(bv, cv, gm);
+            for (int ks = 0; ks < NP / 16; ++ks) {
+                if (ks + 1 < NP / 16) fetch(ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                gm = GD_MFMA(bv[ks & 1], cv[ks & 1], gm); /* (above the diagonal nobody reads it) */
+                ys = GD_MFMA(ah[ks & 1], cv[ks & 1], ys);
+                ys = GD_MFMA(al[ks & 1], cv[ks & 1], ys);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            ys = GD_MFMA(ah, cv, ys);
-            ys = GD_MFMA(al, cv, ys);
         }
         const float ci = s_cs[i];
         __syncthreads(); /* C is used up: M takes its place */
@@ -195,12 +195,12 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
                 const gd_float4 dj = *reinterpret_cast<const gd_float4 *>(&s_dt[j0]);
                 gd_bf16x4 vh, vl;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float v = j0 + (uint32_t)r <= i ? gm[4 * a + r] * __builtin_amdgcn_exp2f(ci - cj[r]) * dj[r] : 0.f;
-                    gd_bf16 hi, lo;
-                    gd_sc_split(v, &hi, &lo);
-                    vh[r] = hi;
-                    vl[r] = lo;
+                for (int r = 0; r < 4; r += 2) {
+                    float v[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        v[e] = j0 + (uint32_t)(r + e) <= i ? gm[4 * a + r + e] * __builtin_amdgcn_exp2f(ci - cj[r + e]) * dj[r + e] : 0.f;
+                    gd_weight_pair(v[0], v[1], vh, vl, r);
                 }
                 *reinterpret_cast<gd_bf16x4 *>(sm + L::mh + i * L::MS + j0 * 2u) = vh;
                 *reinterpret_cast<gd_bf16x4 *>(sm + L::ml + i * L::MS + j0 * 2u) = vl;
@@ -211,15 +211,22 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
             const float ei = __builtin_amdgcn_exp2f(ci);
 #pragma unroll
             for (int e = 0; e < 16; ++e) ys[e] *= ei;
+            gd_bf16x8 xv[2], mh[2], ml[2];
+            auto fetch = [&](int ks) __attribute__((always_inline)) {
+                const uint32_t j = (16u * (uint32_t)ks + 8u * hh) * 2u;
+                xv[ks & 1] = gd_sc_turned(sm + L::x, L::XS, 16u * (uint32_t)ks, 32u * pb, lane);
+                mh[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::mh + i * L::MS + j);
+                ml[ks & 1] = *reinterpret_cast<const gd_bf16x8 *>(sm + L::ml + i * L::MS + j);
+            };
+            fetch(0);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) { /* X^T M^T over j <= i: the second half only for the lower rows */
                 if (16u * ks >= 32u * (ib + 1u)) continue;
-                const uint32_t j = (16u * ks + 8u * hh) * 2u;
-                const gd_bf16x8 xv = gd_sc_turned(sm + L::x, L::XS, 16u * (uint32_t)ks, 32u * pb, lane);
-                const gd_bf16x8 mh = *reinterpret_cast<const gd_bf16x8 *>(sm + L::mh + i * L::MS + j);
-                const gd_bf16x8 ml = *reinterpret_cast<const gd_bf16x8 *>(sm + L::ml + i * L::MS + j);
-                ys = GD_MFMA(xv, mh, ys);
-                ys = GD_MFMA(xv, ml, ys);
+                if (ks + 1 < 4) fetch(ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                ys = GD_MFMA(xv[ks & 1], mh[ks & 1], ys);
+                ys = GD_MFMA(xv[ks & 1], ml[ks & 1], ys);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (i < nt) {
                 gd_bf16 *yr = y + (size_t)(first + t0 + (int32_t)i) * inner + h * P + p0 + 32u * pb;
@@ -246,25 +253,33 @@ gd_ssm_scan_chunk_kernel(const gd_bf16 *__restrict__ xbc, const gd_bf16 *__restr
         for (int tb = 0; tb < TPW; tb += PB) {
             const uint32_t ti = wave * (uint32_t)TPW + (uint32_t)tb, nb = ti / 2u;
             if (ti >= (uint32_t)TILES) continue;
+            gd_bf16x8 bv[2], xv[2][PB];
+            gd_float4 w0[2], w1[2];
+            auto fetch = [&](int ks) __attribute__((always_inline)) {
+                bv[ks & 1] = gd_sc_turned(sm + L::b, L::BC, 16u * (uint32_t)ks, 32u * nb, lane);
+                w0[ks & 1] = *reinterpret_cast<const gd_float4 *>(&s_w[16 * ks + 8 * (int)hh]);
+                w1[ks & 1] = *reinterpret_cast<const gd_float4 *>(&s_w[16 * ks + 8 * (int)hh + 4]);
+#pragma unroll
+                for (int u = 0; u < PB; ++u)
+                    xv[ks & 1][u] = gd_sc_turned(sm + L::x, L::XS, 16u * (uint32_t)ks, 32u * ((ti + (uint32_t)u) % 2u), lane);
+            };
+            fetch(0);
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                const gd_bf16x8 bv = gd_sc_turned(sm + L::b, L::BC, 16u * (uint32_t)ks, 32u * nb, lane);
-                const gd_float4 w0 = *reinterpret_cast<const gd_float4 *>(&s_w[16 * ks + 8 * (int)hh]);
-                const gd_float4 w1 = *reinterpret_cast<const gd_float4 *>(&s_w[16 * ks + 8 * (int)hh + 4]);
+                if (ks + 1 < 4) fetch(ks + 1);
+                __builtin_amdgcn_sched_barrier(0);
                 gd_bf16x8 bh, bl;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    gd_bf16 hi, lo;
-                    gd_sc_split((float)bv[e] * (e < 4 ? w0[e & 3] : w1[e & 3]), &hi, &lo);
-                    bh[e] = hi;
-                    bl[e] = lo;
+                for (int e = 0; e < 8; e += 2) {
+                    const gd_float4 w = e < 4 ? w0[ks & 1] : w1[ks & 1];
+                    gd_weight_pair((float)bv[ks & 1][e] * w[e & 3], (float)bv[ks & 1][e + 1] * w[(e + 1) & 3], bh, bl, e);
                 }
 #pragma unroll
                 for (int u = 0; u < PB; ++u) {
-                    const gd_bf16x8 xv = gd_sc_turned(sm + L::x, L::XS, 16u * (uint32_t)ks, 32u * ((ti + (uint32_t)u) % 2u), lane);
-                    S[tb + u] = GD_MFMA(bh, xv, S[tb + u]);
-                    S[tb + u] = GD_MFMA(bl, xv, S[tb + u]);
+                    S[tb + u] = GD_MFMA(bh, xv[ks & 1][u], S[tb + u]);
+                    S[tb + u] = GD_MFMA(bl, xv[ks & 1][u], S[tb + u]);
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
