@@ -342,7 +342,7 @@ gd_status gd_backend_linear_qkv_rope_packed(gd_backend *backend, const gd_backen
         gd_hip_linear_params tail = p;
         char *work_rows = (char *)gd_hip_matrix_ptr(work) + (size_t)head_rows * work->row_bytes;
         /* the projection of the tail rows in whole 128-row tiles: it starts up to 127 rows early (rows of `work`
-         * nobody reads), so that no ragged row tile leaves the tile kernel's direct staging path */
+         * nobody reads), so that all its row tiles are whole */
         const uint32_t tail_rows = p.M - head_rows;
         const uint32_t up = (tail_rows + 127u) / 128u * 128u;
         const uint32_t first = tail_rows >= 128u && up <= p.M ? p.M - up : head_rows;

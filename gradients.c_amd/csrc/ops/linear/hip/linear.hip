@@ -169,7 +169,7 @@ extern "C" int GD_LINEAR_FN(gd_hip_launch_linear)(hipStream_t stream, const void
         *family = GD_HIP_LINEAR_FAMILY_TILE;
 #if GD_LINEAR_IS_BF16
         /* a last column tile of a few columns (gates, step sizes behind the large parts of a stacked projection) would
-         * take as long as a whole one, and off the direct staging path: the few-row kernel reads x once more instead */
+         * take as long as a whole one: the few-row kernel reads x once more instead */
         const uint32_t narrow = p.N % 256u;
         if (p.swiglu_cols == 0u && p.epilogue == GD_HIP_EPI_NONE && p.N > 256u && narrow != 0u && narrow <= 32u) {
             gd_hip_linear_params rest = p, whole = p;
